@@ -100,19 +100,6 @@ struct LineArgs {
 
 __device__ __forceinline__ int line_swz(int r) { return ((r >> 1) & 3) ^ (((r >> 4) & 1) << 2); }
 
-// v from lane l ^ m of the same 16-lane row (m = 1, 2, 4, 8), through DPP (no LDS): quad
-// permutations for 1 and 2; for 4 and 8 the row shifts up and down, each lane taking the one that
-// reaches its partner.
-template <int m>
-__device__ __forceinline__ float row_xor(float v, int lane) {
-    const int x = __float_as_int(v);
-    if constexpr (m == 1) return __int_as_float(__builtin_amdgcn_update_dpp(x, x, 0xB1, 0xF, 0xF, false));
-    if constexpr (m == 2) return __int_as_float(__builtin_amdgcn_update_dpp(x, x, 0x4E, 0xF, 0xF, false));
-    const int up = __builtin_amdgcn_update_dpp(x, x, 0x100 + m, 0xF, 0xF, false);    // row_shl: lane l + m
-    const int down = __builtin_amdgcn_update_dpp(x, x, 0x110 + m, 0xF, 0xF, false);  // row_shr: lane l - m
-    return __int_as_float((lane & m) ? down : up);
-}
-
 // Four dwords at a 4-byte aligned address, read by one 16-byte load; global-memory pointers to
 // dwords and to such groups (addresses rebuilt from integers would otherwise be flat accesses).
 typedef uint32_t u4a __attribute__((ext_vector_type(4), aligned(4)));

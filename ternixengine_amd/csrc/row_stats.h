@@ -9,6 +9,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <math.h>
+#include <stdint.h>
 
 namespace ternix_hip {
 
@@ -54,6 +55,38 @@ __device__ __forceinline__ float row_absmax(const float* x, const float* w, floa
 __device__ __forceinline__ int quantize_value(float v, float s) {
     const float r = rintf(v * s);
     return (int)fminf(fmaxf(r, -128.0f), 127.0f);
+}
+
+// v from lane l ^ m of the same 16-lane row (m = 1, 2, 4, 8), through DPP (no LDS): quad
+// permutations for 1 and 2; for 4 and 8 the row shifts up and down, each lane taking the one that
+// reaches its partner.
+template <int m>
+__device__ __forceinline__ float row_xor(float v, int lane) {
+    const int x = __float_as_int(v);
+    if constexpr (m == 1) return __int_as_float(__builtin_amdgcn_update_dpp(x, x, 0xB1, 0xF, 0xF, false));
+    if constexpr (m == 2) return __int_as_float(__builtin_amdgcn_update_dpp(x, x, 0x4E, 0xF, 0xF, false));
+    const int up = __builtin_amdgcn_update_dpp(x, x, 0x100 + m, 0xF, 0xF, false);    // row_shl: lane l + m
+    const int down = __builtin_amdgcn_update_dpp(x, x, 0x110 + m, 0xF, 0xF, false);  // row_shr: lane l - m
+    return __int_as_float((lane & m) ? down : up);
+}
+
+typedef float row_f4 __attribute__((ext_vector_type(4)));
+
+// Maximum over the wave.
+__device__ __forceinline__ float row_wave_max(float v, int lane) {
+    v = fmaxf(v, row_xor<8>(v, lane));
+    v = fmaxf(v, row_xor<4>(v, lane));
+    v = fmaxf(v, row_xor<2>(v, lane));
+    v = fmaxf(v, row_xor<1>(v, lane));
+    const int m = __float_as_int(v);
+    return fmaxf(fmaxf(__int_as_float(__builtin_amdgcn_readlane(m, 0)), __int_as_float(__builtin_amdgcn_readlane(m, 16))),
+                 fmaxf(__int_as_float(__builtin_amdgcn_readlane(m, 32)), __int_as_float(__builtin_amdgcn_readlane(m, 48))));
+}
+
+// Four quantised values packed in element order.
+__device__ __forceinline__ uint32_t quantize_pack(row_f4 v, float s) {
+    return (uint32_t)(quantize_value(v[0], s) & 0xFF) | ((uint32_t)(quantize_value(v[1], s) & 0xFF) << 8) |
+           ((uint32_t)(quantize_value(v[2], s) & 0xFF) << 16) | ((uint32_t)(quantize_value(v[3], s) & 0xFF) << 24);
 }
 
 }  // namespace ternix_hip

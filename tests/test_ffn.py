@@ -146,6 +146,44 @@ def test_gpu_rms_norm_quantize(oracle, shape):
     assert diff.max() <= 1 and (diff > 0).mean() < 1e-3   # only values within rounding of a .5 tie move
 
 
+def rms_np(x, w, eps):
+    """RMSNorm in the device's own order of fp32 operations (thread t sums elements t, t + 256,
+    ... with fused multiply-adds, then a butterfly over 64 threads and the four wave sums)."""
+    m, k = x.shape
+    pad = np.zeros((m, -(-k // 256) * 256), F32)
+    pad[:, :k] = x
+    chains = np.zeros((m, 256), F32)
+    for i in range(pad.shape[1] // 256):  # an fma rounds once: exact product and sum in 64 bits, then fp32
+        v = pad[:, 256 * i:256 * (i + 1)].astype(np.float64)
+        chains = (v * v + chains.astype(np.float64)).astype(F32)
+    t = chains.reshape(m, 4, 64)
+    for off in (32, 16, 8, 4, 2, 1):
+        t = t + t[:, :, np.arange(64) ^ off]
+    red = t[:, :, 0]
+    ss = (red[:, 0] + red[:, 1]) + (red[:, 2] + red[:, 3])
+    inv = F32(1) / np.sqrt(ss / F32(k) + F32(eps))
+    return x * inv[:, None] * w
+
+
+@gpu
+@pytest.mark.parametrize("k", [1, 255, 257, 1024, 1028, 2049, 4096, 4097, 8192, 8193, 16384, 16385])
+def test_gpu_rms_norm_row_widths(oracle, k):
+    """The edges of RMSNorm's register forms and of the loop past them, bit for bit up to the 64-bit stand-in
+    for the fma (a double rounding, at most one unit in the last place of the sum)."""
+    from ternixengine_amd import hip_runtime as hr
+    log(f"[rms_norm widths] k={k}")
+    rng = np.random.default_rng(k)
+    x, w = rng.normal(0, 2, (3, k)).astype(F32), rng.normal(1, 0.2, k).astype(F32)
+    y = rms_np(x, w, 1e-5)
+    np.testing.assert_allclose(tx.rms_norm(x, w, 1e-5), y, rtol=4 * 2.0 ** -24, atol=0)
+    dx, dw, dq, ds = _dev(x), _dev(w), hr.DeviceBuffer(3 * k), hr.DeviceBuffer(12)
+    assert tx._load().ternix_hip_rms_norm_quantize(dq.value, ds.value, dx.value, dw.value, 3, k, 1e-5, None) == 0
+    hr.synchronize()
+    qo, rso = o_quant(oracle, tx.rms_norm(x, w, 1e-5))  # the same row, normalised and quantised separately
+    np.testing.assert_array_equal(dq.download(np.int8, (3, k)), qo)
+    np.testing.assert_array_equal(ds.download(F32, (3,)), rso)
+
+
 def _ffn_weights(rng, h, f):
     t_gu = (rng.integers(0, 10, size=(h, 2 * f)) // 4 - 1).clip(-1, 1).astype(np.int8)
     t_d = (rng.integers(0, 10, size=(f, h)) // 4 - 1).clip(-1, 1).astype(np.int8)

@@ -140,6 +140,26 @@ def test_gpu_quantize_matches_oracle(oracle, shape):
     np.testing.assert_array_equal(rs, rso)
 
 
+@gpu
+@pytest.mark.parametrize("k", [4, 1020, 2048, 2052, 4096, 4100, 8192, 8196, 16388, 32768, 32772])
+@pytest.mark.parametrize("offset", [0, 1])  # floats: X aligned to 16 bytes, or not
+def test_gpu_quantize_row_widths(oracle, k, offset):
+    """The edges of the register forms of the row quantiser, and the loop past and beside them: exact."""
+    from ternixengine_amd import hip_runtime as hr
+    log(f"[quantize widths] k={k} offset={offset}")
+    m = 3
+    x = np.random.default_rng(k).standard_normal((m, k)).astype(F32)
+    x[1] *= 40
+    x[2, -1] = 9.0  # the row's maximum in its last element
+    flat = np.concatenate([np.zeros(offset, F32), x.reshape(-1)])
+    dx, dq, ds = hr.DeviceBuffer.from_array(flat), hr.DeviceBuffer(m * k), hr.DeviceBuffer(4 * m)
+    assert tx._load().ternix_hip_quantize_activations(dx.value + 4 * offset, dq.value, ds.value, m, k, None) == 0
+    hr.synchronize()
+    qo, rso = oracle_quant(oracle, x)
+    np.testing.assert_array_equal(dq.download(np.int8, (m, k)), qo)
+    np.testing.assert_array_equal(ds.download(F32, (m,)), rso)
+
+
 def _mm_oracle(oracle, a, wp, n):
     return oracle.mm("scalar", a, wp, n)
 
