@@ -207,8 +207,9 @@ int ternix_hip_device_count(void);
  *   "gemm_narrow" v0    0 / 1: 64 x 64 GEMM tiles for M <= 64 off / forced
  *   "gemm_generic" v0   1: the generic GEMM for every GEMM call
  *   "gemm_splits" v0    GEMM split-K count forced
- *   "gemm_bm" v0        64 / 128 / 256: GEMM tile height forced
- *   "gemm_gm" v0        row tiles per group in the tile order of the 64/128-row GEMMs
+ *   "gemm_bm" v0,v1     v0 64 / 128: GEMM tile height forced (256: as 128); v1 0-6: tile shape
+ *                       of the 32x32x32 MFMA GEMM forced
+ *   "gemm_gm" v0        row tiles per group in the tile order of the GEMMs
  *   "deep" v0..3        0: no whole-K deep GEMV; else force (strip bytes, waves
  *                       per workgroup, ring slots, splits)
  *   "sk_order" v0       1: release/acquire form of the in-launch split sums

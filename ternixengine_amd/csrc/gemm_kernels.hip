@@ -7,6 +7,7 @@
 #include <stdlib.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "kernel_common.h"
 #include "ternary_kernels.h"
@@ -195,35 +196,6 @@ __global__ __launch_bounds__(GM_THREADS) void gemm_kernel(const int8_t* __restri
         }
 }
 
-// ------------------------------------------------------------------------------------------------
-// Pipelined LDS-tiled GEMM (prefill shapes; K % 128 == 0, NB % 64 == 0, aligned A and W).
-//
-// Workgroup = 8 waves (8/WGN along M x WGN along N) on a BM x 64-byte-column tile (BM x 256
-// outputs); wave tile BM*WGN/8 rows x 64/WGN byte-columns, i.e. m-tiles x 16-byte-column groups x
-// 4 fields of 16x16 MFMA outputs.  Each decoded weight fragment feeds all m-tiles of the wave.
-// K advances in stages of 128 (two MFMA k-steps), NS LDS stages deep.
-//   * A and W both go global -> LDS with direct 16-byte loads (global_load_lds_dwordx4): no
-//     registers held, so NS-1 stages are in flight while one is consumed.  Each wave instruction
-//     fills 64 consecutive 16-byte LDS slots; the bank-conflict swizzles are applied by choosing
-//     which global chunk each lane loads.
-//   * A rows (128 bytes per stage): chunk c of row r at position c ^ ((r/2) % 8), so the 16 rows of
-//     one ds_read_b128 fragment read fall on distinct banks.
-//   * W rows stay row-major (64 bytes = 4 chunks per stage row): chunk c of row r at position
-//     c ^ ((r/2) % 4) ^ ((r/16) % 2).  The first term spreads the 8 rows one 16-lane group reads over
-//     32 banks; the second gives the group of the next 16 rows (the other half of the wave's k-block,
-//     read in the same pass) the other 32 banks (measured: no LDS bank conflicts left).
-//     B fragments are read with ds_read_b64_tr_b8, which transposes bytes within
-//     each 16-lane group: result lane j, byte i = byte (j % 8) of the 8 bytes addressed by lane
-//     2i + j/8.  Lane x addresses k-row (x/2) at byte offset 8*(x%2) of its 16-byte-column group,
-//     so lane q receives byte-column q of 8 consecutive k-rows; two reads give the 16 k-rows of its
-//     MFMA B operand, with no VALU transpose and no transposed stores.
-// Stage s: wait until stage s has landed (vmcnt with a static count: every thread issues the same
-// loads each stage, tails are clamped), raw s_barrier, issue stage s+NS-1, then the MFMAs of stage
-// s.  A buffer is refilled only after the barrier that follows its last read.
-// ------------------------------------------------------------------------------------------------
-
-constexpr int GF_THREADS = 512;
-constexpr int GF_BK = 128;
 constexpr int GF_BNB = 64;
 
 __device__ __forceinline__ int gf_swz_a(int r) { return (r >> 1) & 7; }
@@ -234,210 +206,27 @@ __device__ __forceinline__ int gf_swz_w(int r) { return ((r >> 1) & 3) ^ ((r >> 
 template <int BNB>
 __device__ __forceinline__ int swz_w(int r) { return BNB == 64 ? gf_swz_w(r) : (BNB == 32 ? ((r >> 4) & 1) : 0); }
 
-template <int BM, int WGN, int NS, int BK, bool TILED>
-__global__ __launch_bounds__(GF_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
-void gemm_fast_kernel(const int8_t* __restrict__ A, const uint8_t* __restrict__ B, int32_t* __restrict__ C, int M,
-                      int K, int N, int tiles_n, int k_begin, int k_end, int accumulate, int vec_store,
-                      int k_split, OutScale os) {
-    if (gridDim.y > 1) {  // split-K: this workgroup's k-range, partial tile in slab blockIdx.y
-        k_begin += (int)blockIdx.y * k_split;
-        k_end = min(k_end, k_begin + k_split);
-        C += (size_t)blockIdx.y * (size_t)M * (size_t)N;
-    }
-    constexpr int WGM = 8 / WGN;             // waves along M
-    constexpr int WM = BM / WGM;             // rows per wave
-    constexpr int MT = WM / 16;              // m-tiles per wave
-    constexpr int GT = 4 / WGN;              // 16-byte-column groups per wave
-    constexpr int KS = BK / 64;              // MFMA k-steps per stage
-    constexpr int CPR = BK / 16;             // 16-byte A chunks per row per stage
-    constexpr int A_STAGE = BM * BK;         // bytes
-    constexpr int W_STAGE = BK * GF_BNB;     // bytes
-    constexpr int NA = A_STAGE / 16 / GF_THREADS;  // A loads per thread per stage
-    constexpr int NW = W_STAGE / 16 / GF_THREADS;  // W loads per thread per stage
-    // Separate arrays per stage: the compiler tracks in-flight LDS DMA per array, so reads of one
-    // stage do not wait for loads into the others.
-    __shared__ __attribute__((aligned(16))) int8_t sA0[A_STAGE];
-    __shared__ __attribute__((aligned(16))) int8_t sA1[A_STAGE];
-    __shared__ __attribute__((aligned(16))) int8_t sA2[A_STAGE];
-    __shared__ __attribute__((aligned(16))) int8_t sA3[NS > 3 ? A_STAGE : 16];
-    __shared__ __attribute__((aligned(16))) uint8_t sW0[W_STAGE];
-    __shared__ __attribute__((aligned(16))) uint8_t sW1[W_STAGE];
-    __shared__ __attribute__((aligned(16))) uint8_t sW2[W_STAGE];
-    __shared__ __attribute__((aligned(16))) uint8_t sW3[NS > 3 ? W_STAGE : 16];
-    auto stage_a = [&](int i) -> int8_t* { return i == 0 ? sA0 : (i == 1 ? sA1 : (i == 2 ? sA2 : sA3)); };
-    auto stage_w = [&](int i) -> uint8_t* { return i == 0 ? sW0 : (i == 1 ? sW1 : (i == 2 ? sW2 : sW3)); };
-
-    const int NB = N >> 2;
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave / WGN, wn = wave % WGN;
-    const int q = lane & 15, kb = lane >> 4;
-
-    // Block -> tile, XCD-aware: each XCD gets a contiguous run of tile numbers (xcd_linear).
-    // Grouped order: consecutive tile numbers walk 4 row bands before moving to the next column
-    // band, so each XCD's contiguous run of tiles is a ~4 x 8 block (A read by ~2 XCDs and W by
-    // ~4, instead of W by all 8).
-    int tm, tn;
-    {
-        const int t = xcd_linear(blockIdx.x, gridDim.x);
-        const int tiles_m = gridDim.x / tiles_n;
-        constexpr int GM = 4;
-        const int first_m = (t / (GM * tiles_n)) * GM;
-        const int gm = min(tiles_m - first_m, GM);
-        const int local = t % (GM * tiles_n);
-        tm = first_m + local % gm;
-        tn = local / gm;
-    }
-    const int row0 = tm * BM;
-    const int bc0 = tn * GF_BNB;
-    const int nst = (k_end - k_begin) / BK;  // stages
-
-    // Load geometry.  Instruction p of wave w fills 16-byte slots (p*8 + w)*64 + lane.  32-bit lane
-    // offsets (M*K and K*NB < 2^32, checked by the launcher) from wave-uniform bases.
-    uint32_t a_off[NA];
-#pragma unroll
-    for (int p = 0; p < NA; ++p) {
-        const int slot = (p * 8 + wave) * 64 + lane;
-        const int r = slot / CPR, pos = slot % CPR;
-        const int grow = min(row0 + r, M - 1);  // rows past M load row M-1; never stored
-        a_off[p] = (uint32_t)grow * (uint32_t)K + (uint32_t)(((pos & ~7) | ((pos & 7) ^ gf_swz_a(r))) * 16);
-    }
-    uint32_t w_off[NW];
-#pragma unroll
-    for (int p = 0; p < NW; ++p) {
-        const int slot = (p * 8 + wave) * 64 + lane;
-        const int r = slot >> 2, pos = slot & 3;
-        w_off[p] = TILED ? tile64_offset((bc0 >> 4) + (pos ^ gf_swz_w(r)), r, K >> 6)
-                         : (uint32_t)r * (uint32_t)NB + (uint32_t)(bc0 + (pos ^ gf_swz_w(r)) * 16);
-    }
-    auto issue = [&](int st, int buf) {
-        const int sc = min(st, nst - 1);  // clamped: keeps the per-stage load count static
-        const int8_t* abase = A + k_begin + (size_t)sc * BK;
-        int8_t* adst = stage_a(buf);
-#pragma unroll
-        for (int p = 0; p < NA; ++p) lds_dma16(abase + a_off[p], adst + (p * 8 + wave) * 1024);
-        const uint8_t* wbase = TILED ? B + (size_t)((k_begin + sc * BK) >> 6) * 1024
-                                     : B + (size_t)(k_begin + sc * BK) * (size_t)NB;
-        uint8_t* wdst = stage_w(buf);
-#pragma unroll
-        for (int p = 0; p < NW; ++p) lds_dma16(wbase + w_off[p], wdst + (p * 8 + wave) * 1024);
-    };
-
-    v4i acc[MT][GT][4];
-#pragma unroll
-    for (int t = 0; t < MT; ++t)
-#pragma unroll
-        for (int g = 0; g < GT; ++g)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc[t][g][j] = v4i{0, 0, 0, 0};
-
-    auto compute = [&](int buf) {
-        const int8_t* a_st = stage_a(buf);
-        const uint8_t* w_st = stage_w(buf);
-#pragma unroll
-        for (int kk = 0; kk < KS; ++kk) {
-            v4i a[MT];
-#pragma unroll
-            for (int t = 0; t < MT; ++t) {
-                const int r = wm * WM + t * 16 + q;
-                const int c = kk * 4 + kb;  // chunk; the swizzle permutes within groups of 8
-                a[t] = *reinterpret_cast<const v4i*>(a_st + r * BK + 16 * ((c & ~7) | ((c & 7) ^ gf_swz_a(r))));
-            }
-#pragma unroll
-            for (int g = 0; g < GT; ++g) {
-                const int cg = wn * GT + g;  // 16-byte column group within the tile
-                const int r0 = kk * 64 + kb * 16 + (q >> 1);
-                const int r1 = r0 + 8;
-                uint64_t lo = lds_read_tr8(w_st + r0 * GF_BNB + 16 * (cg ^ gf_swz_w(r0)) + 8 * (q & 1));
-                uint64_t hi = lds_read_tr8(w_st + r1 * GF_BNB + 16 * (cg ^ gf_swz_w(r1)) + 8 * (q & 1));
-                // The wait names the results, so no use of them can be scheduled before it.
-                __asm__ volatile("s_waitcnt lgkmcnt(0)" : "+v"(lo), "+v"(hi));
-                const uint32_t x4[4] = {(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
-                v4i bfr[4];
-#pragma unroll
-                for (int r4 = 0; r4 < 4; ++r4) {
-                    const uint32_t x = x4[r4];
-                    bfr[0][r4] = (int)((x << 6) & 0xC0C0C0C0u);
-                    bfr[1][r4] = (int)((x << 4) & 0xC0C0C0C0u);
-                    bfr[2][r4] = (int)((x << 2) & 0xC0C0C0C0u);
-                    bfr[3][r4] = (int)(x & 0xC0C0C0C0u);
-                }
-#pragma unroll
-                for (int t = 0; t < MT; ++t)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) acc[t][g][j] = mfma_i8(a[t], bfr[j], acc[t][g][j]);
-            }
-        }
-    };
-
-    // Prologue: stages 0 .. NS-2 in flight.
-#pragma unroll
-    for (int p = 0; p < NS - 1; ++p) issue(p, p);
-
-    // h is always a literal at the call sites, so after inlining every buffer index is a constant;
-    // the main loop has no conditions, so the compiler counts the loads in flight exactly as the
-    // waits assume.
-    auto stage = [&](int st, int h) {
-        TX_VMCNT((NS - 2) * (NA + NW));  // stage st has landed (the NS-2 later stages may not)
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_sched_barrier(0);
-        issue(st + NS - 1, (h + NS - 1) % NS);
-        compute(h % NS);
-        TX_LGKMCNT0();  // this stage's LDS reads are done before the next barrier
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    int s = 0;
-    for (; s + NS <= nst; s += NS) {
-        stage(s + 0, 0);
-        stage(s + 1, 1);
-        stage(s + 2, 2);
-        if (NS > 3) stage(s + 3, 3);
-    }
-    if (s + 0 < nst) stage(s + 0, 0);
-    if (s + 1 < nst) stage(s + 1, 1);
-    if (NS > 3 && s + 2 < nst) stage(s + 2, 2);
-    TX_VMCNT(0);  // no LDS DMA may land after the workgroup exits
-
-    // Epilogue: element i of tile (t, g, j) is row 4*kb + i of m-tile t, column 4*(byte-col) + j.
-#pragma unroll
-    for (int t = 0; t < MT; ++t)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int row = row0 + wm * WM + t * 16 + 4 * kb + i;
-            if (row >= M) continue;
-#pragma unroll
-            for (int g = 0; g < GT; ++g) {
-                const int bcol = bc0 + (wn * GT + g) * 16 + q;
-                v4i v = {acc[t][g][0][i] >> 6, acc[t][g][1][i] >> 6, acc[t][g][2][i] >> 6, acc[t][g][3][i] >> 6};
-                if (os.Y) {  // dequantised float output: y = c * (row_scale[row] * w_scale)
-                    store_scaled(os, row, N, 4 * bcol, v, vec_store);
-                    continue;
-                }
-                int32_t* out = C + (size_t)row * (size_t)N + 4 * bcol;
-                if (vec_store) {
-                    if (accumulate) v += *reinterpret_cast<const v4i*>(out);
-                    *reinterpret_cast<v4i*>(out) = v;  // write-back stores (on MI355X, cold: 2048x4096x14336
-                    // 103.9 -> 102.0 us, 4096x8192x28672 673 -> 665 against non-temporal ones; the pipelined
-                    // kernel keeps non-temporal stores, 2048x4096x4096 27.0 against 28.4)
-                } else {
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) out[j] = accumulate ? out[j] + v[j] : v[j];
-                }
-            }
-        }
-}
-
 // ------------------------------------------------------------------------------------------------
-// Software-pipelined variant of the LDS-tiled GEMM.  Same tiles, LDS layouts and DMA as
-// gemm_fast_kernel; the difference is the order of work inside a wave:
+// GEMM on v_mfma_i32_16x16x64_i8: the 64-row tiles of 256 columns (4 waves, 64 x 64 outputs each, two
+// workgroups per CU) and the 64 x 64 tiles of up to 64 rows.  K % BK == 0, aligned A and W.
+//   * A and W both go global -> LDS with direct 16-byte loads (global_load_lds_dwordx4): no registers
+//     held, so NS stages are in flight.  Each wave instruction fills 64 consecutive 16-byte LDS slots; the
+//     bank-conflict swizzles are applied by choosing which global chunk each lane loads.
+//   * A rows (128 bytes per stage): chunk c of row r at position c ^ ((r/2) % 8), so the 16 rows of
+//     one ds_read_b128 fragment read fall on distinct banks.
+//   * W rows stay row-major: 64-byte rows keep chunk c of row r at c ^ ((r/2) % 4) ^ ((r/16) % 2).  The
+//     first term spreads the 8 rows one 16-lane group reads over 32 banks; the second gives the group of
+//     the next 16 rows the other 32 (measured: no LDS bank conflicts left).  B fragments are read with
+//     ds_read_b64_tr_b8, which transposes bytes within each 16-lane group: result lane j, byte i = byte
+//     (j % 8) of the 8 bytes addressed by lane 2i + j/8.  Lane x addresses k-row (x/2) at byte offset
+//     8*(x%2) of its 16-byte-column group, so lane q receives byte-column q of 8 consecutive k-rows; two
+//     reads give the 16 k-rows of its MFMA B operand, with no VALU transpose and no transposed stores.
 //   * every LDS fragment read is inline assembly, so the only LDS waits are the explicit ones;
 //   * the fragments of the next MFMA k-step are read while the MFMAs of the current one run
 //     (two register sets, alternating);
 //   * the stage barrier (stage s+1 landed everywhere, stage s free for reuse) and the DMA issue of
 //     stage s+NS happen before the last k-step's MFMAs of stage s, and the first fragments of
 //     stage s+1 are read right after it, so the MFMA pipe never waits for a fresh stage's reads.
-// NS stages are in flight: NS-1 DMA stages ahead of the one being read.
 // ------------------------------------------------------------------------------------------------
 template <int MT, int GT>
 struct PipeFrag {
@@ -447,7 +236,7 @@ struct PipeFrag {
 
 template <int BM, int WGN, int NS, int BK, int NWV, int BNB, bool TILED, int GM = 4>
 __global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(2)))
-void gemm_pipe_kernel(const int8_t* __restrict__ A, const uint8_t* __restrict__ B, int32_t* __restrict__ C, int M,
+void gemm_pipe16_kernel(const int8_t* __restrict__ A, const uint8_t* __restrict__ B, int32_t* __restrict__ C, int M,
                       int K, int N, int tiles_n, int k_begin, int k_end, int accumulate, int vec_store,
                       int k_split, OutScale os, int group_m) {
     if (gridDim.y > 1) {  // split-K: this workgroup's k-range, partial tile in slab blockIdx.y
@@ -642,6 +431,13 @@ void gemm_pipe_kernel(const int8_t* __restrict__ A, const uint8_t* __restrict__ 
     if (s + 0 < nst) stage(s + 0, 0);
     if (s + 1 < nst) stage(s + 1, 1);
     if (NS > 3 && s + 2 < nst) stage(s + 2, 2);
+    float fs[MT][4];  // the float epilogue's row scales, all in flight at once
+    if (os.Y) {
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) fs[t][i] = os.rs[min(row0 + wm * WM + t * 16 + 4 * kb + i, M - 1)];
+    }
     TX_VMCNT(0);  // no LDS DMA may land after the workgroup exits
 
 #pragma unroll
@@ -655,7 +451,7 @@ void gemm_pipe_kernel(const int8_t* __restrict__ A, const uint8_t* __restrict__ 
                 const int bcol = bc0 + (wn * GT + g) * 16 + q;
                 v4i v = {acc[t][g][0][i] >> 6, acc[t][g][1][i] >> 6, acc[t][g][2][i] >> 6, acc[t][g][3][i] >> 6};
                 if (os.Y) {  // dequantised float output: y = c * (row_scale[row] * w_scale)
-                    store_scaled(os, row, N, 4 * bcol, v, vec_store);
+                    store_scaled_f(os, fs[t][i] * os.ws, row, N, 4 * bcol, v, vec_store);
                     continue;
                 }
                 int32_t* out = C + (size_t)row * (size_t)N + 4 * bcol;
@@ -668,6 +464,372 @@ void gemm_pipe_kernel(const int8_t* __restrict__ A, const uint8_t* __restrict__ 
                 }
             }
         }
+}
+
+// ------------------------------------------------------------------------------------------------
+// GEMM on v_mfma_i32_32x32x32_i8 (K % 16 == 0, K >= BK, NB % 16 == 0, aligned A and W; output columns n_out <= N).
+//
+// A workgroup is WGM x WGN x WGK waves; a wave computes 32*MT rows x 32 byte-columns (128 outputs), MT x 4
+// accumulators of 32x32, over its share of every stage's k-rows.  What bounds it, on MI355X:
+//   * Prefill (every CU full): power.  The clock falls to 1.85-2.15 GHz with the MFMA pipes 79 % busy; from
+//     registers alone 32x32x32 sustains 4.34 POPS, 16x16x64 3.9.  So the tile spends little energy beside the
+//     MFMAs: it is wide in N, since a packed weight byte is four columns (64 x 128 outputs read 64 + 32 bytes of
+//     LDS per k-row where a 64 x 64 tile reads 64 + 16 for half the work).
+//   * Fewer tiles than CUs: issue.  One wave per SIMD ran at 61 % (decode 17 %, DMA 14 %, barriers 11 %), so the
+//     smaller tiles split each stage's k-steps over WGK waves, which sum their tiles through LDS at the end:
+//     no partial sums in memory, no second launch, and two or more waves on every SIMD.
+// Each MFMA is followed by a share of the other work, so that the pipe always has the next one: half a field of
+// the next decode, two of the next k-step's LDS reads (first MFMAs), one or two of the stage's DMAs (its last
+// k-step).  DMAs in one burst after the barrier cost 6 % (1024x6912x2560 24.0 -> 22.0 us).
+// us before -> after, L2-warm weights: 128x4096x4096 19.3 -> 9.5, 256x4096x11008 20.7 -> 16.7, 1024x6912x2560 31.4 ->
+// 22.1, 1024x2560x13824 41 -> 34.5, 2048x4096x14336 126 -> 111 (the card at its slowest; 103 -> 98 otherwise).
+// LDS layouts (no bank conflicts): A chunk c of row r at c ^ ((r/2) % 8) for 128-byte rows, c ^ (r % 16) for
+// 256-byte ones; W's 32-byte column pairs p of row r at p ^ f(r), f the row bits that make 8 rows of one pair
+// cover all 64 banks.  W fragments come from ds_read_b64_tr_b8 (see below): 16-lane groups 0-1 take the two
+// halves of a pair for k-rows 0-15, groups 2-3 for rows 16-31, as the MFMA's lanes want them.
+// ------------------------------------------------------------------------------------------------
+typedef int v16i __attribute__((ext_vector_type(16)));
+
+template <int BK>
+__device__ __forceinline__ int gw_swz_a(int r) { return BK == 128 ? ((r >> 1) & 7) : (r & 15); }
+template <int BNB>
+__device__ __forceinline__ int gw_swz_w(int r) {
+    return BNB == 128 ? 2 * ((r >> 1) & 3) : (BNB == 64 ? 2 * ((r >> 2) & 1) : 0);
+}
+
+template <int OFF>
+__device__ __forceinline__ v4i lds_read_b128_off(uint32_t addr) {
+    v4i v;
+    __asm__ volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
+    return v;
+}
+template <int OFF>
+__device__ __forceinline__ uint64_t lds_read_tr8_off(uint32_t addr) {
+    uint64_t v;
+    __asm__ volatile("ds_read_b64_tr_b8 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
+    return v;
+}
+
+template <int V>
+using Int = std::integral_constant<int, V>;
+
+template <int MT>
+struct WideFrag {
+    v4i a[MT];
+    uint64_t lo, hi;
+};
+
+template <int WGM, int WGN, int WGK, int MT, int BK, int NS, bool TILED, int GM>
+__global__ __launch_bounds__(64 * WGM * WGN * WGK) __attribute__((amdgpu_waves_per_eu(2)))
+void gemm_pipe_kernel(const int8_t* __restrict__ A, const uint8_t* __restrict__ B, int32_t* __restrict__ C, int M,
+                      int K, int N, int n_out, int tiles_n, int k_begin, int k_end, int accumulate, int vec_store,
+                      int k_split, OutScale os, int group_m) {
+    if (gridDim.y > 1) {  // split-K: this workgroup's k-range, partial tile in slab blockIdx.y
+        k_begin += (int)blockIdx.y * k_split;
+        k_end = min(k_end, k_begin + k_split);
+        C += (size_t)blockIdx.y * (size_t)M * (size_t)n_out;
+    }
+    constexpr int NWV = WGM * WGN * WGK;
+    constexpr int THR = 64 * NWV;
+    constexpr int BM = 32 * MT * WGM;
+    constexpr int BNB = 32 * WGN;
+    constexpr int CW = BNB / 16;           // 16-byte chunks per W stage row
+    constexpr int CPR = BK / 16;           // and per A stage row
+    constexpr int KS = BK / 32 / WGK;      // 32-row k-steps per wave and stage
+    constexpr int A_STAGE = BM * BK;
+    constexpr int W_STAGE = BK * BNB;
+    constexpr int STAGE = A_STAGE + W_STAGE;
+    constexpr int NA = A_STAGE / 16 / THR;
+    constexpr int NW = W_STAGE / 16 / THR;
+    constexpr int RED = WGK == 1 ? 0 : NWV * (WGK - 1) * (16 / WGK) * 1024;  // bytes of the final exchange
+    constexpr int LDS = NS * STAGE > RED ? NS * STAGE : RED;
+    static_assert(KS == 2 || KS == 4, "fragment sets alternate per k-step");
+    static_assert(NA >= 1 && NW >= 1 && A_STAGE % (16 * THR) == 0 && W_STAGE % (16 * THR) == 0, "uneven stage");
+    static_assert(LDS <= 160 * 1024, "LDS");
+    __shared__ __attribute__((aligned(256))) uint8_t smem[LDS];
+
+    const int NB = N >> 2;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wk = wave / (WGM * WGN), wmn = wave % (WGM * WGN);
+    const int wm = wmn / WGN, wn = wmn % WGN;
+    const int r32 = lane & 31, half = lane >> 5, q = lane & 15;
+
+    const int tiles_m = (M + BM - 1) / BM;
+    int tm, tn;
+    {
+        const int t = xcd_linear(blockIdx.x, gridDim.x);
+        const int G_M = group_m > 0 ? group_m : GM;  // row tiles per group of the tile order
+        const int first_m = (t / (G_M * tiles_n)) * G_M;
+        const int gm = min(tiles_m - first_m, G_M);
+        const int local = t % (G_M * tiles_n);
+        tm = first_m + local % gm;
+        tn = local / gm;
+    }
+    const int row0 = tm * BM;
+    const int bc0 = tn * BNB;
+    // Stages of BK k-rows; the last one ends at k_end, so where BK does not divide the range it starts inside
+    // the stage before, and the rows that one has done are masked out of its weights.
+    const int klen = k_end - k_begin;
+    const int nst = (klen + BK - 1) / BK;
+    const int done = nst * BK - klen;  // k-rows of the last stage that the stage before it has done
+
+    uint32_t a_off[NA];
+#pragma unroll
+    for (int p = 0; p < NA; ++p) {
+        const int slot = (p * NWV + wave) * 64 + lane;
+        const int r = slot / CPR, pos = slot % CPR;
+        const int grow = min(row0 + r, M - 1);  // rows past M load row M-1; never stored
+        a_off[p] = (uint32_t)grow * (uint32_t)K + (uint32_t)((pos ^ gw_swz_a<BK>(r)) * 16);
+    }
+    uint32_t w_off[NW];
+#pragma unroll
+    for (int p = 0; p < NW; ++p) {
+        const int slot = (p * NWV + wave) * 64 + lane;
+        const int r = slot / CW, pos = slot % CW;
+        const int c = min((bc0 >> 4) + (pos ^ gw_swz_w<BNB>(r)), (NB >> 4) - 1);  // columns past N: never stored
+        w_off[p] = TILED ? tile64_offset(c, r, K >> 6) : (uint32_t)r * (uint32_t)NB + (uint32_t)(c * 16);
+    }
+    // DMA instruction d of stage st (A's NA, then W's NW) into the stage buffer at byte `off`.
+    // (Stages past the last one repeat it: the load count per stage stays static, and a branch around the
+    // loads cost more than the repeats.)
+    auto issue = [&](int st, int off, int d) {
+        const int k0 = k_begin + min(st * BK, klen - BK);
+        if (d < NA) {
+            lds_dma16(A + k0 + a_off[d < NA ? d : 0], smem + off + (d * NWV + wave) * 1024);
+        } else {
+            const int p = d - NA;
+            const uint8_t* wbase = TILED ? B + (size_t)(k0 >> 6) * 1024 : B + (size_t)k0 * (size_t)NB;
+            lds_dma16(wbase + w_off[p < 0 ? 0 : p], smem + off + A_STAGE + (p * NWV + wave) * 1024);
+        }
+    };
+
+    uint32_t a_lane[KS];
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk) {
+        const int r = wm * MT * 32 + r32;
+        const int c = (wk * KS + kk) * 2 + half;
+        a_lane[kk] = lds_u32(smem) + (uint32_t)(r * BK + 16 * (c ^ gw_swz_a<BK>(r)));
+    }
+    const uint32_t w_lane = lds_u32(smem) + (uint32_t)(((wk * KS * 32) + half * 16 + (q >> 1)) * BNB +
+                                       16 * ((2 * wn + ((lane >> 4) & 1)) ^ gw_swz_w<BNB>(q >> 1)) + 8 * (q & 1));
+    // Read r (0, 1: the weights' halves; 2 ..: m-tile r - 2) of k-step KK of the stage at byte `off`.
+    auto read = [&](auto kc, WideFrag<MT>& f, uint32_t off, int r) {
+        constexpr int KK = decltype(kc)::value;
+        if (r == 0) f.lo = lds_read_tr8_off<A_STAGE + KK * 32 * BNB>(w_lane + off);
+        if (r == 1) f.hi = lds_read_tr8_off<A_STAGE + KK * 32 * BNB + 8 * BNB>(w_lane + off);
+        if (r == 2) f.a[0] = lds_read_b128_off<0>(a_lane[KK] + off);
+        if constexpr (MT > 1)
+            if (r == 3) f.a[1] = lds_read_b128_off<32 * BK>(a_lane[KK] + off);
+    };
+    // The reads still outstanding may be the MT youngest (the activations); tie the registers to the wait.
+    auto wait_w = [&](WideFrag<MT>& f) {
+        __builtin_amdgcn_s_waitcnt(0xF | (3 << 14) | (7 << 4) | (MT << 8));
+        __asm__ volatile("" : "+v"(f.lo), "+v"(f.hi));
+    };
+    auto wait_a = [&](WideFrag<MT>& f) {
+        TX_LGKMCNT0();
+#pragma unroll
+        for (int t = 0; t < MT; ++t) __asm__ volatile("" : "+v"(f.a[t]));
+    };
+
+    v16i acc[MT][4];
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[t][j][i] = 0;
+
+    // Field mask of each k-step: all fields, or none in the last stage's steps that are already done (a lane
+    // holds 16 consecutive k-rows of a step, and every k-range is a multiple of 16 rows).
+    auto field_mask = [&](bool last, int kk) -> uint32_t {
+        return last && (wk * KS + kk) * 32 + half * 16 < done ? 0u : 0xC0C0C0C0u;
+    };
+    uint32_t mask[KS];
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk) mask[kk] = field_mask(nst == 1, kk);
+    v4i b0, b1;                         // decoded fields: one feeds the MFMAs while the next one is made
+    auto decode = [&](v4i& b, const WideFrag<MT>& f, int j, int r4, uint32_t m) {
+        const uint32_t x = r4 == 0 ? (uint32_t)f.lo : (r4 == 1 ? (uint32_t)(f.lo >> 32)
+                                                               : (r4 == 2 ? (uint32_t)f.hi : (uint32_t)(f.hi >> 32)));
+        b[r4] = (int)((j == 3 ? x : x << (6 - 2 * j)) & m);
+    };
+    constexpr int D = NA + NW;      // DMA instructions per stage
+    constexpr int SLOTS = 4 * MT;   // MFMAs per k-step
+    constexpr int R = 2 + MT;       // LDS reads per k-step
+
+    WideFrag<MT> f0, f1;
+#pragma unroll
+    for (int p = 0; p < NS; ++p)
+#pragma unroll
+        for (int d = 0; d < D; ++d) issue(p, p * STAGE, d);
+    TX_VMCNT((NS - 1) * D);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int r = 0; r < R; ++r) read(Int<0>{}, f0, 0, r);
+    wait_w(f0);
+#pragma unroll
+    for (int r4 = 0; r4 < 4; ++r4) decode(b0, f0, 0, r4, mask[0]);
+    wait_a(f0);
+
+    // One 32-row k-step: SLOTS MFMAs, each followed by a share of the next field's decode, of the next
+    // k-step's LDS reads (first half) and, in a stage's last k-step, of the DMAs of stage st + NS.
+    auto step = [&](auto kc, WideFrag<MT>& cur, WideFrag<MT>& nxt, int st, uint32_t off, uint32_t noff) {
+        constexpr int KK = decltype(kc)::value;
+        constexpr bool LAST = KK + 1 == KS;
+        if constexpr (LAST) {
+            // stage st + 1 has landed (the NS - 2 later ones may not)
+            TX_VMCNT((NS - 2) * D);
+            __builtin_amdgcn_s_barrier();  // ... everywhere, and every wave is done reading stage st
+        }
+        if (LAST && done > 0 && st + 2 == nst) {
+#pragma unroll
+            for (int kk = 0; kk + 1 < KS; ++kk) mask[kk] = field_mask(true, kk);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < SLOTS; ++s) {
+            const int j = s / MT, t = s % MT;
+            v4i& b = (j & 1) ? b1 : b0;
+            v4i& bn = (j & 1) ? b0 : b1;
+            acc[t][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(cur.a[t], b, acc[t][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            if (s == 3 * MT) wait_w(nxt);
+#pragma unroll
+            for (int r4 = t * 4 / MT; r4 < (t + 1) * 4 / MT; ++r4)
+                decode(bn, j == 3 ? nxt : cur, (j + 1) & 3, r4, mask[j == 3 ? (KK + 1) % KS : KK]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                if (r / 2 == s) read(Int<(KK + 1) % KS>{}, nxt, LAST ? noff : off, r);
+            if constexpr (LAST) {
+#pragma unroll
+                for (int d = 0; d < D; ++d)
+                    if (d * SLOTS / D == s) issue(st + NS, (int)off, d);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        wait_a(nxt);
+        if (LAST && done > 0 && st + 2 == nst) mask[KS - 1] = field_mask(true, KS - 1);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    uint32_t off = 0;
+    for (int st = 0; st < nst; ++st) {
+        const uint32_t noff = off + STAGE == (uint32_t)(NS * STAGE) ? 0u : off + STAGE;
+        step(Int<0>{}, f0, f1, st, off, noff);
+        step(Int<1>{}, f1, f0, st, off, noff);
+        if constexpr (KS == 4) {
+            step(Int<2>{}, f0, f1, st, off, noff);
+            step(Int<3>{}, f1, f0, st, off, noff);
+        }
+        off = noff;
+    }
+    // The float epilogue's row scales, all in flight at once (loaded one by one between the stores they cost a
+    // memory latency per row: dequantising 1024x2560x13824 38.3 us against 34 for int32).
+    float fs[MT][16];
+    if (os.Y) {
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                fs[t][i] = os.rs[min(row0 + (wm * MT + t) * 32 + 8 * (i >> 2) + 4 * half + (i & 3), M - 1)];
+    }
+    TX_VMCNT(0);  // no LDS DMA may land after the workgroup exits
+
+    // Element i of accumulator (t, j) is row 8*(i/4) + 4*half + i%4 of m-tile t, column 4*r32 + j.
+    auto store = [&](int t, int i, v4i v) {
+        const int row = row0 + (wm * MT + t) * 32 + 8 * (i >> 2) + 4 * half + (i & 3);
+        const int bcol = bc0 + wn * 32 + r32;
+        if (row >= M || bcol >= (n_out >> 2)) return;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] >>= 6;
+        if (os.Y) {  // dequantised float output: y = c * (row_scale[row] * w_scale)
+            store_scaled_f(os, fs[t][i] * os.ws, row, n_out, 4 * bcol, v, vec_store);
+            return;
+        }
+        int32_t* out = C + (size_t)row * (size_t)n_out + 4 * bcol;
+        if (vec_store) {
+            if (accumulate) v += *reinterpret_cast<const v4i*>(out);
+            __builtin_nontemporal_store(v, reinterpret_cast<v4i*>(out));  // streamed, not re-read
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) out[j] = accumulate ? out[j] + v[j] : v[j];
+        }
+    };
+    if constexpr (WGK == 1) {
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) store(t, i, v4i{acc[t][0][i], acc[t][1][i], acc[t][2][i], acc[t][3][i]});
+    } else {
+        // Each of the WGK waves of one output tile finishes 1/WGK of its elements: per m-tile it leaves the
+        // other shares in LDS for their owners and adds what they left for it.
+        constexpr int SH = 16 / WGK;  // elements i per share and m-tile
+        v4i* ex = reinterpret_cast<v4i*>(smem);  // [wmn][owner][sender slot][SH][64 lanes]
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int owner = i / SH;
+                const int slot = (wk - owner + WGK) % WGK - 1;  // 0 .. WGK-2 for the other waves
+                if (owner != wk)
+                    ex[(((wmn * WGK + owner) * (WGK - 1) + slot) * SH + i % SH) * 64 + lane] =
+                        v4i{acc[t][0][i], acc[t][1][i], acc[t][2][i], acc[t][3][i]};
+            }
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int owner = i / SH;
+                if (owner != wk) continue;
+                v4i v = {acc[t][0][i], acc[t][1][i], acc[t][2][i], acc[t][3][i]};
+#pragma unroll
+                for (int sl = 0; sl < WGK - 1; ++sl)
+                    v += ex[(((wmn * WGK + owner) * (WGK - 1) + sl) * SH + i % SH) * 64 + lane];
+                store(t, i, v);
+            }
+        }
+    }
+}
+
+// Tile shapes of gemm_pipe_kernel and what they cost (gemm_plan).  us per 256 k-rows of a round: t1 with one
+// workgroup on every CU, t2 with per_cu of them; one_cu of t1 on an idle chip; second of the way to t2 where
+// the first CUs get a second workgroup.  fixed + a round's start and stores.
+struct WideTile {
+    int rows, bnb, bk, per_cu;
+    float t1, t2, fixed, round, second, one_cu;
+};
+// Fitted to 5800 timings of 228 shapes (M 33-2048, K 512-16384, N 768-16384, 1-16 splits; root mean square error
+// 7 %); the plans it picks are within 1 % of the fastest of these tiles on average.
+constexpr WideTile kWide[kWideTiles] = {
+    {32, 32, 256, 2, 0.455f, 0.872f, 1.96f, 2.57f, 0.674f, 0.60f},   // 0: 32 x 128, K over 4 waves
+    {32, 64, 256, 2, 0.550f, 1.31f, 0.00f, 4.88f, 0.862f, 0.681f},   // 1: 32 x 256, K over 4 of 8 waves
+    {64, 64, 256, 1, 0.708f, 0.811f, 2.36f, 4.66f, 1.0f, 0.672f},    // 2: 64 x 256, K over 4 of 8 waves
+    {64, 128, 128, 1, 1.34f, 1.60f, 1.89f, 4.65f, 1.0f, 0.698f},     // 3: 64 x 512, K over 2 of 8 waves
+    {64, 128, 128, 2, 1.56f, 3.25f, 2.02f, 4.23f, 0.409f, 0.736f},   // 4: 64 x 512, 4 waves, two workgroups per CU
+    {64, 64, 128, 2, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f},            // 5: 64 x 256, K over 2 of 4 waves (split plans)
+    {128, 64, 128, 1, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f},           // 6: 128 x 256, K over 2 of 8 waves (split plans)
+};
+// The 64 x 256 tiles of gemm_pipe16_kernel, on the same scale.
+constexpr WideTile kPipe64Cost = {64, 64, 128, 2, 1.08f, 1.76f, 0.001f, 4.75f, 0.225f, 0.732f};
+
+template <int WGM, int WGN, int WGK, int MT, int BK, int NS, int GM>
+hipError_t launch_wide(const int8_t* A, const uint8_t* B, int32_t* C, int M, int K, int N, int n_out, int kb, int ke,
+                       int acc, int vs, hipStream_t st, const OutScale& os, int splits, int k_split, int tiled,
+                       int gm_env) {
+    constexpr int BM = 32 * MT * WGM, BNB = 32 * WGN;
+    const int tiles_n = (N / 4 + BNB - 1) / BNB;
+    const dim3 grid((unsigned)(((M + BM - 1) / BM) * tiles_n), splits), block(64 * WGM * WGN * WGK);
+    if (tiled)
+        hipLaunchKernelGGL((gemm_pipe_kernel<WGM, WGN, WGK, MT, BK, NS, true, GM>), grid, block, 0, st, A, B, C, M, K, N,
+                           n_out, tiles_n, kb, ke, acc, vs, k_split, os, gm_env);
+    else
+        hipLaunchKernelGGL((gemm_pipe_kernel<WGM, WGN, WGK, MT, BK, NS, false, GM>), grid, block, 0, st, A, B, C, M, K, N,
+                           n_out, tiles_n, kb, ke, acc, vs, k_split, os, gm_env);
+    return hipGetLastError();
 }
 
 template <int BM, int BNB>
@@ -707,10 +869,6 @@ bool gemm_narrow_wanted(int M, int K, int N, int tiled) {
     return (long)((M + 63) / 64) * (NB / 16) <= device_cu_count();
 }
 
-bool gemm_narrow_ok(int M, int K, int N, int k_len, int splits, int k_split, int tiled) {
-    return gemm_narrow_wanted(M, K, N, tiled) && k_len % 256 == 0 && (splits == 1 || k_split % 256 == 0);
-}
-
 // Tile height of a split-K launch: 64-row tiles of four waves or 128-row tiles of eight, each with
 // the split count sized to one workgroup per CU (at most 16 splits of >= 256 k-rows).  The plan that
 // keeps more CUs busy wins; on a tie the 64-row tiles win where they need no split at all on a full
@@ -740,106 +898,203 @@ int gemm_split_rows(int M, int K, int N) {
     return macs >= 80e6 ? 128 : 64;
 }
 
-// Which GEMM kernel a launch_gemm call runs (the single place the choice is made).
-GemmChoice gemm_choice(const int8_t* A, const uint8_t* B, int M, int K, int N, int k_begin, int k_end, int splits,
-                       int k_split, int tiled) {
+namespace {
+
+// Predicted us of one launch over `len` k-rows (and of the reduce launch with splits > 1).
+double wide_cost(const WideTile& w, long M, long N, long len, long splits) {
+    const long cus = device_cu_count(), slots = cus * w.per_cu;
+    const long wgs = ((M + w.rows - 1) / w.rows) * ((N / 4 + w.bnb - 1) / w.bnb) * splits;
+    const long full = wgs / slots, rem = wgs % slots;
+    double last = 0.0;
+    if (rem > cus) last = w.t1 + (w.t2 - w.t1) * (w.second + (1.0 - w.second) * (double)(rem - cus) / (double)cus);
+    else if (rem > 0) last = w.t1 * (w.one_cu + (1.0 - w.one_cu) * (double)rem / (double)cus);
+    double t = w.fixed + (double)(full + (rem > 0)) * w.round + (double)len / 256.0 * ((double)full * w.t2 + last);
+    if (splits > 1) t += 2.5 + (0.787 * (double)splits + 0.621) * (double)M * (double)N * 1e-6;
+    return t;
+}
+
+// K over `splits` ranges of whole 64-row blocks, none shorter than `least` rows; fewer where they do not fit.
+void split_k(int K, long splits, int least, GemmPlan* p) {
+    for (; splits > 1; --splits) {
+        const int ks = (int)((K / splits + (K % splits != 0) + 63) / 64 * 64);
+        const int n = (K + ks - 1) / ks;
+        if (n > 1 && K - (n - 1) * ks >= least) {
+            p->splits = n;
+            p->k_split = ks;
+            return;
+        }
+    }
+    p->splits = 1;
+    p->k_split = 0;
+}
+
+// The split count of the row-tile plan (gemm_split_rows): one workgroup per CU, at most 16 splits of >= 256 rows.
+int row_tile_splits(int M, int K, int N, int bm, int col_tiles) {
+    // K <= 4096: the reduce launch and the partial sums cost more than the idle CUs (measured on
+    // MI355X, cold weights: 40x1024x4096 7.6 -> 4.9 us without the split, 64x2560x6912 11.8 -> 8.8,
+    // 256x1024x11008 31.1 -> 9.7, 256x4096x11008 35.2 -> 25.0; from K = 6144 the split wins:
+    // 128x11008x4096 59.0 -> 22.4 us).
+    if (K <= 4096) return 1;
+    const long tiles = (long)((M + bm - 1) / bm) * col_tiles, cus = device_cu_count();
+    return (int)std::max<long>(1, std::min<long>({tiles * 2 <= cus ? cus / tiles : 1, (long)K / 256, 16L}));
+}
+
+}  // namespace
+
+// Which kernel a GEMM call runs and how it splits K (the single place the choice is made).
+GemmPlan gemm_plan(const int8_t* A, const uint8_t* B, int M, int K, int N, int tiled, bool may_split, bool padded) {
+    GemmPlan p;
     const int NB = N >> 2;
+    const bool aligned = (uintptr_t)A % 16 == 0 && (uintptr_t)B % 16 == 0 && (size_t)M * (size_t)K < ((size_t)1 << 32) &&
+                         (size_t)512 * (size_t)NB < ((size_t)1 << 32) && M > 0;
     const bool force_generic = debug_get(DBG_GEMM_GENERIC) == 1;  // tests
-    if (splits < 1) splits = 1;
-    const bool fast = (K % GF_BK == 0) && ((k_end - k_begin) % GF_BK == 0) && (k_begin % GF_BK == 0) &&
-                      (splits == 1 || k_split % GF_BK == 0) &&
-                      (NB % GF_BNB == 0) && ((uintptr_t)A % 16 == 0) && ((uintptr_t)B % 16 == 0) &&
-                      k_end > k_begin && (size_t)M * (size_t)K < ((size_t)1 << 32) &&
-                      (size_t)GF_BK * (size_t)NB < ((size_t)1 << 32) &&
+    const bool pipe16 = aligned && !padded && K > 0 && K % 128 == 0 && NB % 64 == 0 && (tiled || !force_generic);
+    const bool wide = aligned && K >= 128 && K % 16 == 0 && NB % 16 == 0 && (!tiled || K % 64 == 0) &&
                       (tiled || !force_generic);
     // The tile-64 layout is read by the LDS-DMA GEMMs only (whole 128-row stages, at most 4 GiB of W).
-    if (tiled && (!fast || (size_t)K * (size_t)NB >= ((size_t)1 << 32))) return GemmChoice::Invalid;
-    if (!fast) return GemmChoice::Generic;
-    const int tiles_n = NB / GF_BNB;
-    const int bm_env = debug_get(DBG_GEMM_BM);
-    // Measured on MI355X (cfg4 shapes): 256-row tiles only when they still give >= 1.5 tiles per
-    // CU, else 128-row tiles; 8 waves as 2 (M) x 4 (N); 128-deep stages.
-    const int cus = device_cu_count();
-    int bm = (splits == 1 && (long)((M + 255) / 256) * tiles_n * 2 >= 3L * cus) ? 256 : 128;
-    if (bm_env > 0) bm = bm_env == 128 ? 128 : (bm_env == 64 ? 64 : 256);  // tests and measurements
-    constexpr int small_m_max = 64;
+    if (tiled && (!pipe16 || (size_t)K * (size_t)NB >= ((size_t)1 << 32))) {
+        p.choice = GemmChoice::Invalid;
+        return p;
+    }
+    const int splits_env = debug_get(DBG_GEMM_SPLITS);  // tests
+    auto forced = [&](long s) { return splits_env > 0 ? (long)splits_env : s; };
+    if (!pipe16 && !wide) {
+        if (may_split) split_k(K, forced(row_tile_splits(M, K, N, gemm_split_rows(M, K, N), (NB + 63) / 64)), 64, &p);
+        return p;  // Generic
+    }
     // 64 x 64 output tiles (16 bytes of every weight row): enough workgroups without a K split where
     // the 256-column tiles would need one; one m-tile per wave, 256-deep stages.
-    if ((M <= small_m_max || debug_get(DBG_GEMM_NARROW) > 0) && gemm_narrow_ok(M, K, N, k_end - k_begin, splits, k_split, tiled)) return GemmChoice::Narrow64;
-    // Without a K split, 64-row tiles in workgroups of four waves (two co-resident per CU, whose
-    // barriers and final stores overlap each other's work) instead of 128-row tiles of eight waves:
-    // measured on MI355X, cold weights, 2048x4096x4096 29.1 -> 27.6 us, 1024x4096x4096 25.4 -> 20.3,
-    // 512x4096x4096 25.1 -> 19.5, 768x4096x11008 52.2 -> 46.1, 1536x4096x11008 81.2 -> 71.7,
-    // 2048x14336x4096 90.6 -> 90.4 (one round: equal).  With a K split: gemm_split_rows.  Small M (64
-    // rows or fewer): the same four-wave workgroups, so no MFMA row or A byte is spent on padding
-    // rows; the caller splits K to fill the chip.
-    const bool split64 = splits > 1 && bm_env <= 0 && gemm_split_rows(M, K, N) == 64;
-    if (M <= small_m_max || bm == 64 || split64 || (splits == 1 && bm == 128 && bm_env <= 0))
-        return GemmChoice::Pipe64;
-    return bm == 128 ? GemmChoice::Pipe128 : GemmChoice::Fast256;
+    if (pipe16 && (M <= 64 || debug_get(DBG_GEMM_NARROW) > 0) && gemm_narrow_wanted(M, K, N, tiled)) {
+        p.choice = GemmChoice::Narrow64;
+        long s = forced(row_tile_splits(M, K, N, 64, NB / 16));
+        if (may_split && s > 1) {  // whole 256-row stages
+            p.k_split = (int)((K + s - 1) / s + 255) / 256 * 256;
+            p.splits = (K + p.k_split - 1) / p.k_split;
+        }
+        return p;
+    }
+    auto use_wide = [&](int i, long s) {
+        p.choice = (GemmChoice)((int)GemmChoice::Wide0 + i);
+        if (may_split) split_k(K, s, kWide[i].bk, &p);
+    };
+    auto use_pipe64 = [&](long s) {
+        p.choice = GemmChoice::Pipe64;
+        if (may_split && s > 1) {  // whole 128-row stages
+            p.k_split = (int)((K + s - 1) / s + 127) / 128 * 128;
+            p.splits = (K + p.k_split - 1) / p.k_split;
+        }
+    };
+    const int bm_env = debug_get(DBG_GEMM_BM), tile_env = debug_get(DBG_GEMM_BM, 1);  // tests and measurements
+    if (wide && tile_env >= 0 && tile_env < kWideTiles && K >= kWide[tile_env].bk) {
+        use_wide(tile_env, forced(1));
+        return p;
+    }
+    const int bm = gemm_split_rows(M, K, N);
+    const long rows_splits = forced(row_tile_splits(M, K, N, bm, (NB + 63) / 64));
+    if (bm_env > 0) {
+        if (bm_env == 64 && pipe16) use_pipe64(rows_splits);
+        else if (wide) use_wide(bm_env == 64 ? 5 : 6, rows_splits);
+        else use_pipe64(rows_splits);
+        return p;
+    }
+    // Four or more splits above 64 rows keep the tile height and the split count of gemm_split_rows, which
+    // the plan descriptions promise; the model below would pick 5-16 % faster plans there (512x11008x4096
+    // 32.0 against 28.4 us, 256x8192x2048 15.4 against 13.5).  128-row tiles are tile 6 (against eight waves
+    // of 64 x 64: 512x11008x4096 33.9 -> 32.0, 512x16384x4096 46.1 -> 39.3), 64-row ones tile 5 from 1024 k-rows a
+    // split (256x16384x4096 28.4 -> 25.5, 256x11008x4096 23.0 -> 21.6; shorter ranges stay, 128x6912x2560 13.0
+    // against 13.9).
+    if (M > 64 && pipe16 && rows_splits >= 4 && may_split) {
+        if (bm == 128) use_wide(6, rows_splits);
+        else if (K / rows_splits >= 1024) use_wide(5, rows_splits);
+        else use_pipe64(rows_splits);
+        return p;
+    }
+    // gemm_pipe16_kernel's tiles take what is within 7 % of a tie: they are level or ahead there (2048x4096x4096 30.4
+    // against 32.0 us, 512x2560x13824 20.3 / 21.3, 512x4096x11008 25.9 / 27.7), on every other choice behind.
+    const long cus = device_cu_count();
+    double best = pipe16 ? 0.93 * wide_cost(kPipe64Cost, M, N, K, 1) : 1e30;
+    int tile = -1;
+    long splits = 1;
+    for (int i = 0; wide && i < 5; ++i) {
+        if (K < kWide[i].bk) continue;
+        const long tiles = (long)((M + kWide[i].rows - 1) / kWide[i].rows) * (long)((NB + kWide[i].bnb - 1) / kWide[i].bnb);
+        for (const long s : {1L, 2L, 3L, 4L, 6L, 8L, 12L, 16L}) {
+            // a split where K is long, each range at least 512 rows, and up to two rounds of two per CU
+            if (s > 1 && (!may_split || K <= 4096 || K / s < 512 || tiles * s > 4 * cus)) break;
+            const double t = wide_cost(kWide[i], M, N, (K + s - 1) / s, s);
+            if (t < best) best = t, tile = i, splits = s;
+        }
+    }
+    if (tile < 0) use_pipe64(1);
+    else use_wide(tile, forced(splits));
+    if (splits_env > 0 && tile < 0) use_pipe64(splits_env);
+    return p;
 }
 
 const char* gemm_choice_name(GemmChoice c) {
     switch (c) {
-        case GemmChoice::Narrow64: return "gemm_pipe_kernel<64 rows x 64 cols, 4 waves>";
-        case GemmChoice::Pipe64: return "gemm_pipe_kernel<64 rows x 256 cols, 4 waves>";
-        case GemmChoice::Pipe128: return "gemm_pipe_kernel<128 rows x 256 cols, 8 waves>";
-        case GemmChoice::Fast256: return "gemm_fast_kernel<256 rows x 256 cols, 8 waves>";
+        case GemmChoice::Narrow64: return "gemm_pipe_kernel<64 rows x 64 cols, 4 waves, 16x16x64>";
+        case GemmChoice::Pipe64: return "gemm_pipe_kernel<64 rows x 256 cols, 4 waves, 16x16x64>";
+        case GemmChoice::Wide0: return "gemm_pipe_kernel<32 rows x 128 cols, K over 4 waves>";
+        case GemmChoice::Wide1: return "gemm_pipe_kernel<32 rows x 256 cols, K over 4 of 8 waves>";
+        case GemmChoice::Wide2: return "gemm_pipe_kernel<64 rows x 256 cols, K over 4 of 8 waves>";
+        case GemmChoice::Wide3: return "gemm_pipe_kernel<64 rows x 512 cols, K over 2 of 8 waves>";
+        case GemmChoice::Wide4: return "gemm_pipe_kernel<64 rows x 512 cols, 4 waves>";
+        case GemmChoice::Wide5: return "gemm_pipe_kernel<64 rows x 256 cols, K over 2 of 4 waves>";
+        case GemmChoice::Wide6: return "gemm_pipe_kernel<128 rows x 256 cols, K over 2 of 8 waves>";
         case GemmChoice::Generic: return "gemm_kernel<128 rows x 256 cols, register-staged>";
         default: return "invalid";
     }
 }
 
-hipError_t launch_gemm(const int8_t* A, const uint8_t* B, int32_t* C, int M, int K, int N, int k_begin, int k_end,
-                       int accumulate, hipStream_t st, const OutScale& os, int splits, int k_split, int tiled) {
-    const int NB = N >> 2;
-    if (splits < 1) splits = 1;
-    const GemmChoice choice = gemm_choice(A, B, M, K, N, k_begin, k_end, splits, k_split, tiled);
-    if (choice == GemmChoice::Invalid) return hipErrorInvalidValue;
-    if (choice == GemmChoice::Generic) {
-        const bool aw = (NB % 4 == 0) && ((uintptr_t)B % 4 == 0);
-        const bool aa = (K % 16 == 0) && ((uintptr_t)A % 16 == 0);
-        return launch_gemm_t<128, 64>(A, B, C, M, K, N, aw, aa, k_begin, k_end, accumulate, st, os, splits, k_split);
-    }
+hipError_t launch_gemm(const GemmPlan& p, const int8_t* A, const uint8_t* B, int32_t* C, int M, int K, int N, int k_begin,
+                       int k_end, int accumulate, hipStream_t st, const OutScale& os, int tiled, int n_out) {
+    const int NB = N >> 2, splits = p.splits, k_split = p.k_split;
+    if (n_out <= 0) n_out = N;
     const int vs = ((uintptr_t)(os.Y ? (const void*)os.Y : (const void*)C) % 16) == 0;
     const int tiles_n = NB / GF_BNB;
     const int gm_env = std::max(0, debug_get(DBG_GEMM_GM));  // tests and measurements: tile-order group
-    if (choice == GemmChoice::Narrow64) {
-        const dim3 gridn((unsigned)(((M + 63) / 64) * (NB / 16)), splits);
-        if (tiled)
-            hipLaunchKernelGGL((gemm_pipe_kernel<64, 1, 3, 256, 4, 16, true>), gridn, dim3(256), 0, st, A, B, C, M, K,
-                               N, NB / 16, k_begin, k_end, accumulate, vs, k_split, os, gm_env);
-        else
-            hipLaunchKernelGGL((gemm_pipe_kernel<64, 1, 3, 256, 4, 16, false>), gridn, dim3(256), 0, st, A, B, C, M,
-                               K, N, NB / 16, k_begin, k_end, accumulate, vs, k_split, os, gm_env);
-    } else if (choice == GemmChoice::Pipe64) {
-        // Tiles are visited in groups of 8 row tiles per column band (512 rows, as 4 groups of 128-row
-        // tiles): measured on MI355X with cold weights, 2048x4096x4096 28.4 -> 27.0 us against groups of 4.
-        const dim3 grid64((unsigned)(((M + 63) / 64) * tiles_n), splits);
-        if (tiled)
-            hipLaunchKernelGGL((gemm_pipe_kernel<64, 4, 3, 128, 4, 64, true, 8>), grid64, dim3(256), 0, st, A, B, C,
-                               M, K, N, tiles_n, k_begin, k_end, accumulate, vs, k_split, os, gm_env);
-        else
-            hipLaunchKernelGGL((gemm_pipe_kernel<64, 4, 3, 128, 4, 64, false, 8>), grid64, dim3(256), 0, st, A, B, C,
-                               M, K, N, tiles_n, k_begin, k_end, accumulate, vs, k_split, os, gm_env);
-    } else if (choice == GemmChoice::Pipe128) {
-        const dim3 grid(((M + 127) / 128) * tiles_n, splits);
-        if (tiled)
-            hipLaunchKernelGGL((gemm_pipe_kernel<128, 4, 3, 128, 8, GF_BNB, true>), grid, dim3(GF_THREADS), 0, st, A,
-                               B, C, M, K, N, tiles_n, k_begin, k_end, accumulate, vs, k_split, os, gm_env);
-        else
-            hipLaunchKernelGGL((gemm_pipe_kernel<128, 4, 3, 128, 8, GF_BNB, false>), grid, dim3(GF_THREADS), 0, st, A,
-                               B, C, M, K, N, tiles_n, k_begin, k_end, accumulate, vs, k_split, os, gm_env);
-    } else {
-        const dim3 grid(((M + 255) / 256) * tiles_n, splits);
-        if (tiled)
-            hipLaunchKernelGGL((gemm_fast_kernel<256, 4, 3, 128, true>), grid, dim3(GF_THREADS), 0, st, A, B, C, M, K,
-                               N, tiles_n, k_begin, k_end, accumulate, vs, k_split, os);
-        else
-            hipLaunchKernelGGL((gemm_fast_kernel<256, 4, 3, 128, false>), grid, dim3(GF_THREADS), 0, st, A, B, C, M,
-                               K, N, tiles_n, k_begin, k_end, accumulate, vs, k_split, os);
+    if (n_out != N && p.choice < GemmChoice::Wide0) return hipErrorInvalidValue;
+#define TX_WIDE(...) \
+    launch_wide<__VA_ARGS__>(A, B, C, M, K, N, n_out, k_begin, k_end, accumulate, vs, st, os, splits, k_split, tiled, gm_env)
+    switch (p.choice) {
+        case GemmChoice::Invalid: return hipErrorInvalidValue;
+        case GemmChoice::Generic: {
+            const bool aw = (NB % 4 == 0) && ((uintptr_t)B % 4 == 0);
+            const bool aa = (K % 16 == 0) && ((uintptr_t)A % 16 == 0);
+            return launch_gemm_t<128, 64>(A, B, C, M, K, N, aw, aa, k_begin, k_end, accumulate, st, os, splits, k_split);
+        }
+        case GemmChoice::Narrow64: {
+            const dim3 gridn((unsigned)(((M + 63) / 64) * (NB / 16)), splits);
+            if (tiled)
+                hipLaunchKernelGGL((gemm_pipe16_kernel<64, 1, 3, 256, 4, 16, true>), gridn, dim3(256), 0, st, A, B, C, M,
+                                   K, N, NB / 16, k_begin, k_end, accumulate, vs, k_split, os, gm_env);
+            else
+                hipLaunchKernelGGL((gemm_pipe16_kernel<64, 1, 3, 256, 4, 16, false>), gridn, dim3(256), 0, st, A, B, C,
+                                   M, K, N, NB / 16, k_begin, k_end, accumulate, vs, k_split, os, gm_env);
+            return hipGetLastError();
+        }
+        case GemmChoice::Pipe64: {
+            // Tiles are visited in groups of 8 row tiles per column band (512 rows): measured on MI355X with
+            // cold weights, 2048x4096x4096 28.4 -> 27.0 us against groups of 4.
+            const dim3 grid64((unsigned)(((M + 63) / 64) * tiles_n), splits);
+            if (tiled)
+                hipLaunchKernelGGL((gemm_pipe16_kernel<64, 4, 3, 128, 4, 64, true, 8>), grid64, dim3(256), 0, st, A, B,
+                                   C, M, K, N, tiles_n, k_begin, k_end, accumulate, vs, k_split, os, gm_env);
+            else
+                hipLaunchKernelGGL((gemm_pipe16_kernel<64, 4, 3, 128, 4, 64, false, 8>), grid64, dim3(256), 0, st, A, B,
+                                   C, M, K, N, tiles_n, k_begin, k_end, accumulate, vs, k_split, os, gm_env);
+            return hipGetLastError();
+        }
+        case GemmChoice::Wide0: return TX_WIDE(1, 1, 4, 1, 256, 4, 8);
+        case GemmChoice::Wide1: return TX_WIDE(1, 2, 4, 1, 256, 3, 8);
+        case GemmChoice::Wide2: return TX_WIDE(1, 2, 4, 2, 256, 4, 8);
+        case GemmChoice::Wide3: return TX_WIDE(1, 4, 2, 2, 128, 4, 8);
+        case GemmChoice::Wide4: return TX_WIDE(1, 4, 1, 2, 128, 3, 8);
+        case GemmChoice::Wide5: return TX_WIDE(1, 2, 2, 2, 128, 3, 8);
+        default: return TX_WIDE(2, 2, 2, 2, 128, 4, 4);
     }
-    return hipGetLastError();
+#undef TX_WIDE
 }
 
 }  // namespace ternix_hip

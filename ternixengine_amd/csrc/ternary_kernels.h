@@ -38,7 +38,7 @@ enum DebugKey : int {
     DBG_GEMM_NARROW,     // [0] 0 / 1: 64 x 64 GEMM tiles for M <= 64 off / forced
     DBG_GEMM_GENERIC,    // [0] == 1: the generic (register-staged) GEMM for every GEMM call
     DBG_GEMM_SPLITS,     // [0] GEMM split-K count forced
-    DBG_GEMM_BM,         // [0] 64 / 128 / 256: GEMM tile height forced
+    DBG_GEMM_BM,         // [0] 64 / 128: GEMM tile height forced (256: as 128); [1] gemm_pipe_kernel tile forced (0-6)
     DBG_DEEP,            // [0] == 0: no whole-K deep GEMV; else (sw, nw, nsw, splits) forced
     DBG_SK_ORDER,        // [0] 1: release/acquire (agent scope) for the in-launch split sums
     DBG_M1_ATOMIC,       // [0] 0: no zero-fill + atomic split plan for M = 1 GEMVs; [1] / [2] largest M of
@@ -154,19 +154,26 @@ hipError_t launch_skinny_wave(const int8_t* A, const uint8_t* B, int32_t* C, int
 bool gemm_narrow_wanted(int M, int K, int N, int tiled = 0);
 // Tile height (64 or 128 rows) launch_gemm uses for this shape when K is split.
 int gemm_split_rows(int M, int K, int N);
-// The GEMM kernel launch_gemm runs for these arguments (Invalid: it would return hipErrorInvalidValue).
-enum class GemmChoice { Invalid, Narrow64, Pipe64, Pipe128, Fast256, Generic };
-GemmChoice gemm_choice(const int8_t* A, const uint8_t* B, int M, int K, int N, int k_begin, int k_end, int splits,
-                       int k_split, int tiled);
+// The GEMM kernel of a call and its K split.  Wide0 ..: gemm_pipe_kernel's tile shapes.
+enum class GemmChoice { Invalid, Generic, Narrow64, Pipe64, Wide0, Wide1, Wide2, Wide3, Wide4, Wide5, Wide6 };
+constexpr int kWideTiles = 7;
+struct GemmPlan {
+    GemmChoice choice = GemmChoice::Generic;
+    int splits = 1, k_split = 0;
+};
+// may_split: partial sums can be written ([splits][M][n_out] int32); else one split.  padded: the output has
+// fewer columns than N, which only gemm_pipe_kernel stores (the others through slabs of N columns).
+GemmPlan gemm_plan(const int8_t* A, const uint8_t* B, int M, int K, int N, int tiled, bool may_split,
+                   bool padded = false);
 const char* gemm_choice_name(GemmChoice c);
 // LDS-tiled MFMA GEMM over k-rows [k_begin, k_end); accumulate != 0 adds into C instead of storing.
 // With os.Y set the tile epilogue writes the dequantised floats instead (accumulate must be 0).
-// splits > 1: split-K over gridDim.y, each workgroup row of the grid covering k_split k-rows (a
-// multiple of 64, of 128 for the fast kernels) and writing its partial tile to C + y * M * N
-// (accumulate must be 0 and os unset; launch_splitk_reduce finishes the sum).
-hipError_t launch_gemm(const int8_t* A, const uint8_t* B, int32_t* C, int M, int K, int N, int k_begin,
-                       int k_end, int accumulate, hipStream_t st, const OutScale& os = OutScale{}, int splits = 1,
-                       int k_split = 0, int tiled = 0);
+// p.splits > 1: split-K over gridDim.y, each workgroup row of the grid covering p.k_split k-rows and writing its
+// partial tile to C + y * M * n_out (accumulate must be 0 and os unset; launch_splitk_reduce finishes the sum).
+// n_out > 0 (Wide tiles only): a padded problem, C / os.Y has n_out <= N columns.
+hipError_t launch_gemm(const GemmPlan& p, const int8_t* A, const uint8_t* B, int32_t* C, int M, int K, int N,
+                       int k_begin, int k_end, int accumulate, hipStream_t st, const OutScale& os = OutScale{},
+                       int tiled = 0, int n_out = 0);
 // (tiled != 0: W in the tile-64 layout; needs K % 128 == 0, N/4 % 64 == 0, aligned operands, k-ranges
 // of whole 128-row stages, K * N/4 < 2^32; hipErrorInvalidValue otherwise.)
 // C (or os.Y) = sum over `splits` slabs of P ([splits][M][N] int32).

@@ -784,60 +784,42 @@ hipError_t run_skinny(const int8_t* dA, const uint8_t* dB, int32_t* dC, int M, i
     return TX_LAUNCH(c, ternix_hip::launch_skinny(dA, dB, dC, M, K, N, p.tb, p.kw, p.splits, p.sps, partials, st, os, aq, p.dma));
 }
 
-// Split-K for GEMMs with too few output tiles to fill the chip (mid-size M against a long K, e.g.
-// cfg3 M=64, the worst case M=256): each split covers a contiguous k-range of whole 128-row stages,
-// the partial tiles go through the same workspace and reduce launch as the skinny path.
-int gemm_splits(int M, int K, int N, int tiled = 0) {
-    const int env = ternix_hip::debug_get(ternix_hip::DBG_GEMM_SPLITS);  // tests
-    // the tile height launch_gemm picks for a split launch; one workgroup per CU over the tiles and
-    // splits
-    const bool narrow = ternix_hip::gemm_narrow_wanted(M, K, N, tiled);  // 64-column tiles instead of 256
-    const int bm = narrow ? 64 : ternix_hip::gemm_split_rows(M, K, N);
-    const long tiles = (long)((M + bm - 1) / bm) * (long)((N / 4 + 63) / 64) * (narrow ? 4 : 1);
-    const long cus = cu_count();
-    // K <= 4096: the reduce launch and the partial sums cost more than the idle CUs (measured on
-    // MI355X, cold weights: 40x1024x4096 7.6 -> 4.9 us without the split, 64x2560x6912 11.8 -> 8.8,
-    // 256x1024x11008 31.1 -> 9.7, 256x4096x11008 35.2 -> 25.0; from K = 6144 the split wins:
-    // 128x11008x4096 59.0 -> 22.4 us).
-    if (env <= 0 && K <= 4096) return 1;
-    long splits = env > 0 ? env : (tiles * 2 <= cus ? cus / tiles : 1);
-    splits = std::min<long>(splits, std::max(1, K / 256));  // at least two 128-row stages per split
-    return (int)std::max<long>(1, std::min<long>(splits, 16));
-}
-
+// GEMMs: gemm_plan picks the kernel and its K split (few output tiles against a long K); partial tiles of a
+// split go through the same workspace and reduce launch as the skinny path.
 hipError_t run_gemm(const int8_t* dA, const uint8_t* dB, int32_t* dC, int M, int K, int N, Ctx& c,
                     const ternix_hip::OutScale& os = ternix_hip::OutScale{}, int tiled = 0) {
     const hipStream_t st = c.st;
     (void)st;
+    using ternix_hip::GemmChoice;
+    using ternix_hip::GemmPlan;
     if (K <= ternix_hip::kMaxKPerAccumulator) {
-        int splits = gemm_splits(M, K, N, tiled);
-        if (splits > 1) {
-            // whole stages per split: 256 rows for the narrow tiles, 128 for the others
-            const int unit = ternix_hip::gemm_narrow_wanted(M, K, N, tiled) ? 256 : (K % 128 == 0 ? 128 : 64);
-            const int k_split = ((K + splits - 1) / splits + unit - 1) / unit * unit;
-            splits = (K + k_split - 1) / k_split;
-            const size_t need = (size_t)splits * (size_t)M * (size_t)N * sizeof(int32_t);
-            int32_t* partials = (splits > 1 && need <= kWorkspaceMax) ? static_cast<int32_t*>(c.get(need))
-                                                                       : nullptr;
+        GemmPlan p = ternix_hip::gemm_plan(dA, dB, M, K, N, tiled, true);
+        if (p.splits > 1) {
+            const size_t need = (size_t)p.splits * (size_t)M * (size_t)N * sizeof(int32_t);
+            int32_t* partials = need <= kWorkspaceMax ? static_cast<int32_t*>(c.get(need)) : nullptr;
             if (partials) {
-                c.note("%s splits=%d + splitk_reduce_kernel",
-                       ternix_hip::gemm_choice_name(ternix_hip::gemm_choice(dA, dB, M, K, N, 0, K, splits, k_split, tiled)),
-                       splits);
-                hipError_t e = TX_LAUNCH(c, ternix_hip::launch_gemm(dA, dB, partials, M, K, N, 0, K, 0, st, ternix_hip::OutScale{},
-                                                       splits, k_split, tiled));
+                c.note("%s splits=%d + splitk_reduce_kernel", ternix_hip::gemm_choice_name(p.choice), p.splits);
+                hipError_t e = TX_LAUNCH(c, ternix_hip::launch_gemm(p, dA, dB, partials, M, K, N, 0, K, 0, st,
+                                                                    ternix_hip::OutScale{}, tiled));
                 if (e != hipSuccess) return e;
-                return TX_LAUNCH(c, ternix_hip::launch_splitk_reduce(partials, dC, M, N, splits, os, st));
+                return TX_LAUNCH(c, ternix_hip::launch_splitk_reduce(partials, dC, M, N, p.splits, os, st));
             }
+            p = ternix_hip::gemm_plan(dA, dB, M, K, N, tiled, false);
         }
-        c.note("%s", ternix_hip::gemm_choice_name(ternix_hip::gemm_choice(dA, dB, M, K, N, 0, K, 1, 0, tiled)));
-        return TX_LAUNCH(c, ternix_hip::launch_gemm(dA, dB, dC, M, K, N, 0, K, 0, st, os, 1, 0, tiled));
+        c.note("%s", ternix_hip::gemm_choice_name(p.choice));
+        return TX_LAUNCH(c, ternix_hip::launch_gemm(p, dA, dB, dC, M, K, N, 0, K, 0, st, os, tiled));
     }
     if (dC == nullptr) return hipErrorInvalidValue;  // scaled call without int scratch
     int acc = 0;
     for (long k0 = 0; k0 < K; k0 += ternix_hip::kMaxKPerAccumulator) {
         const long k1 = k0 + ternix_hip::kMaxKPerAccumulator < K ? k0 + ternix_hip::kMaxKPerAccumulator : K;
-        const hipError_t e = TX_LAUNCH(c, ternix_hip::launch_gemm(dA, dB, dC, M, K, N, (int)k0, (int)k1, acc, st,
-                                                     ternix_hip::OutScale{}, 1, 0, tiled));
+        GemmPlan p = ternix_hip::gemm_plan(dA, dB, M, K, N, tiled, false);
+        // A chunk is a multiple of 128 rows but not of 256, and the last one may be short: tiles of 128-row
+        // stages there, the generic kernel below one stage (never tile-64 weights, whose K % 128 == 0).
+        if (p.choice == GemmChoice::Narrow64) p.choice = GemmChoice::Pipe64;
+        if (p.choice >= GemmChoice::Wide0) p.choice = k1 - k0 >= 128 ? GemmChoice::Wide5 : GemmChoice::Generic;
+        const hipError_t e = TX_LAUNCH(c, ternix_hip::launch_gemm(p, dA, dB, dC, M, K, N, (int)k0, (int)k1, acc, st,
+                                                                  ternix_hip::OutScale{}, tiled));
         if (e != hipSuccess) return e;
         acc = 1;
     }
@@ -863,7 +845,8 @@ hipError_t run_padded(const int8_t* dA, const uint8_t* dB, int32_t* dC, int M, i
     const long Np = 4 * NBp;
     if (K == 0 || Kp > INT_MAX || Np > INT_MAX || Kp * NBp >= (1L << 32)) return hipErrorNotSupported;
     SkinnyPlan p{0, 0, 0, 0, 0};
-    int splits = 1, k_split = 0;
+    int splits = 1;
+    ternix_hip::GemmPlan g;
     // Short K at M <= 16: the wave-pipelined kernel in one launch, writing the N real columns itself.
     const bool wave = skinny && M <= kWaveMaxM && Kp <= 4096 && wave_kernel_enabled();
     if (wave) {
@@ -873,26 +856,28 @@ hipError_t run_padded(const int8_t* dA, const uint8_t* dB, int32_t* dC, int M, i
         if (p.dma == 0) p = plan_skinny(M, (int)Kp, (int)Np);
         splits = p.splits;
     } else {
-        splits = gemm_splits(M, (int)Kp, (int)Np);
-        if (splits > 1) {
-            const long unit = ternix_hip::gemm_narrow_wanted(M, (int)Kp, (int)Np) ? 256 : 128;
-            k_split = (int)(((Kp + splits - 1) / splits + unit - 1) / unit * unit);
-            splits = (int)((Kp + k_split - 1) / k_split);
-        }
+        // (aligned by construction: the copies are 256-byte aligned)
+        g = ternix_hip::gemm_plan(reinterpret_cast<const int8_t*>(uintptr_t(4096)), reinterpret_cast<const uint8_t*>(uintptr_t(4096)),
+                                  M, (int)Kp, (int)Np, 0, true, true);
+        splits = g.splits;
+        if ((splits > 1 ? g.k_split : Kp) > ternix_hip::kMaxKPerAccumulator) return hipErrorNotSupported;  // int32 sums
     }
-    // The skinny kernels write partials only through a split; the GEMM writes its one slab to the
-    // workspace just the same, and the reduce launch keeps the N real columns.
+    // gemm_pipe_kernel's tiles write the N real columns themselves: into C without a split, else into slabs of
+    // N columns; the generic kernel (forced) writes Np columns to one or more slabs, of which the reduce keeps N.
+    const bool real_cols = !skinny && g.choice >= ternix_hip::GemmChoice::Wide0;
+    const bool direct = real_cols && splits == 1;
+    // The skinny kernels write partials only through a split.
     if (splits <= 1 && skinny && !wave) return hipErrorNotSupported;
-    // Each split's k-range must fit one int32 accumulator (the skinny plans guarantee it).
-    if (!skinny && k_split > ternix_hip::kMaxKPerAccumulator) return hipErrorNotSupported;
     auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
     const size_t w_bytes = up((size_t)Kp * (size_t)NBp);
     const size_t a_bytes = up((size_t)M * (size_t)Kp);
-    const size_t p_bytes = wave ? 0 : (size_t)splits * (size_t)M * (size_t)Np * sizeof(int32_t);
+    const size_t p_bytes = wave || direct ? 0 : (size_t)splits * (size_t)M * (size_t)(real_cols ? N : Np) * sizeof(int32_t);
     if (w_bytes + a_bytes + p_bytes > kWorkspaceMax) return hipErrorNotSupported;
     uint8_t* ws = static_cast<uint8_t*>(c.get(w_bytes + a_bytes + p_bytes));
     if (ws == nullptr) return hipErrorNotSupported;
-    c.note("pad_rows_kernel + %s", wave ? "skinny_wave_kernel" : (skinny ? (p.dma ? "skinny_dma_kernel" : "skinny_short/fast_kernel") : "gemm"));
+    c.note("pad_rows_kernel + %s", wave ? "skinny_wave_kernel"
+                                        : (skinny ? (p.dma ? "skinny_dma_kernel" : "skinny_short/fast_kernel")
+                                                  : ternix_hip::gemm_choice_name(g.choice)));
     uint8_t* Wp = ws;
     int8_t* Ap = reinterpret_cast<int8_t*>(ws + w_bytes);
     int32_t* P = reinterpret_cast<int32_t*>(ws + w_bytes + a_bytes);
@@ -912,17 +897,20 @@ hipError_t run_padded(const int8_t* dA, const uint8_t* dB, int32_t* dC, int M, i
     if (skinny)
         return TX_LAUNCH(c, ternix_hip::launch_skinny(Ap, Wp, dC, M, (int)Kp, (int)Np, p.tb, p.kw, p.splits, p.sps, P, st, os,
                                          ternix_hip::ActQuant{}, p.dma, N));
-    e = TX_LAUNCH(c, ternix_hip::launch_gemm(Ap, Wp, P, M, (int)Kp, (int)Np, 0, (int)Kp, 0, st, ternix_hip::OutScale{}, splits,
-                                k_split));
+    if (direct)
+        return TX_LAUNCH(c, ternix_hip::launch_gemm(g, Ap, Wp, dC, M, (int)Kp, (int)Np, 0, (int)Kp, 0, st, os, 0, N));
+    e = TX_LAUNCH(c, ternix_hip::launch_gemm(g, Ap, Wp, P, M, (int)Kp, (int)Np, 0, (int)Kp, 0, st, ternix_hip::OutScale{}, 0,
+                                             real_cols ? N : 0));
     if (e != hipSuccess) return e;
-    return TX_LAUNCH(c, ternix_hip::launch_splitk_reduce(P, dC, M, N, splits, os, st, (int)Np));
+    return TX_LAUNCH(c, ternix_hip::launch_splitk_reduce(P, dC, M, N, splits, os, st, real_cols ? N : (int)Np));
 }
 
-// The aligned kernels need 16-byte aligned operands, N/4 % 64 == 0 and whole k-steps: 64 rows for
-// the skinny kernels, 128 for the pipelined GEMM.
+// The aligned kernels need 16-byte aligned operands and, the skinny ones, N/4 % 64 == 0 and whole 64-row
+// k-steps; the GEMMs whole 128-row stages and N/4 % 64 == 0, or, from 256 k-rows, any rows of whole 16-byte chunks.
 bool needs_padding(const int8_t* dA, const uint8_t* dB, int K, int N, bool skinny) {
-    return !(K % (skinny ? 64 : 128) == 0 && (N / 4) % 64 == 0 && reinterpret_cast<uintptr_t>(dB) % 16 == 0 &&
-             reinterpret_cast<uintptr_t>(dA) % 16 == 0);
+    const bool sizes = skinny ? K % 64 == 0 && (N / 4) % 64 == 0
+                              : (K % 128 == 0 && (N / 4) % 64 == 0) || (K % 16 == 0 && K >= 256 && (N / 4) % 16 == 0);
+    return !(sizes && reinterpret_cast<uintptr_t>(dB) % 16 == 0 && reinterpret_cast<uintptr_t>(dA) % 16 == 0);
 }
 
 // Automatic path for one call: the padded copy for ragged or misaligned shapes when it applies,
