@@ -311,16 +311,17 @@ int ternix_hip_rms_norm_quantize(int8_t* dQ, float* dRowScale, const float* dIn,
 /* Up-projection with dequantisation and SwiGLU fused into its output: the N output columns
  * are interleaved (gate, up) pairs, dH is M x N/2 fp32 with
  *   dH[m][i] = silu(y[m][2i]) * y[m][2i+1],  y = (float)C * (dRowScale[m] * w_scale).
- * dScratch (M x N int32, may be NULL) is used only when the split-K or K-chunk path cannot
- * fuse the epilogue (first use of a shape inside graph capture, K > 131008); such a call
- * with dScratch == NULL returns hipErrorInvalidValue. */
+ * dScratch (M x N int32, may be NULL) holds the int32 sums where a second launch finishes them (few rows:
+ * faster, and without it another plan runs) and where the split-K or K-chunk path cannot fuse the
+ * epilogue (first use of a shape inside graph capture, K > 131008); such a call with dScratch == NULL
+ * returns hipErrorInvalidValue. */
 int ternix_hip_mul_mat_ternary_swiglu(const int8_t* dA, const uint8_t* dB, float* dH, int64_t M, int64_t K,
                                       int64_t N, const float* dRowScale, float w_scale, int32_t* dScratch,
                                       void* stream);
 /* Bytes of device workspace ternix_hip_ffn_forward needs for M rows, hidden size H and
  * intermediate size F. */
 size_t ternix_hip_ffn_workspace_size(int64_t M, int64_t H, int64_t F);
-/* One BitNet-style feed-forward block, four launches on `stream`:
+/* One BitNet-style feed-forward block on `stream`, as if by four launches:
  *   q1, rs1 = rms_norm_quantize(dX, dNormWeight, eps)                  [M x H]
  *   h       = swiglu matmul(q1, dWgu: H x 2F packed, interleaved gate/up columns, ws_gu)
  *   q2, rs2 = quantize_activations(h)                                  [M x F]

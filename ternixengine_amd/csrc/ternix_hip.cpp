@@ -913,6 +913,23 @@ bool needs_padding(const int8_t* dA, const uint8_t* dB, int K, int N, bool skinn
     return !(sizes && reinterpret_cast<uintptr_t>(dB) % 16 == 0 && reinterpret_cast<uintptr_t>(dA) % 16 == 0);
 }
 
+// Up to 32 rows on aligned operands there are two ways: the GEMVs (K split over the chip; an int32 C gets the
+// splits with atomics, a float output partial sums and a reduce) and gemm_pipe_kernel's 32-row tiles (K split
+// over the waves of a workgroup, any epilogue in the same launch, few workgroups on a narrow N).  Estimates in us, least-squares fits to 28 (K, N) pairs x 2-32 rows measured warm on
+// MI355X (rms error 4-5 %, 8 % for few_rows_float_us); choosing by them is within 1 % of the best of the measured
+// times.  mb: packed weights in MB, mn: outputs in millions.
+double few_rows_gemm_us(int K, double mb) {  // 32-row tiles (nearly the same for 1 and 32 rows)
+    return 3.43 + 5.58 * std::min(K, 4096) / 4096.0 + 0.171 * std::max(K - 4096, 0) / 4096.0 + 0.133 * mb;
+}
+double few_rows_gemv_us(int M, int K, double mb, double mn) {  // int32 GEMVs of 4-16 / 17-32 rows
+    return M <= 16 ? 3.69 + 0.191 * mb - 1.76 * mn + 0.1296 * M + 0.0026 * M * mb
+                   : 5.39 + 0.195 * mb + 1.30 * mn + 0.003 * M + 0.81 * K / 8192.0 + 0.0044 * M * mb;
+}
+double few_rows_float_us(int M, int K, double mb, double mn) {  // the GEMVs' float outputs
+    if (M <= 16) return few_rows_gemv_us(M, K, mb, mn) + 2.0;
+    return 7.0 + 0.332 * mb - 8.91 * mn + 0.0576 * M - 0.52 * K / 8192.0 + 0.00675 * M * mb;
+}
+
 // Automatic path for one call: the padded copy for ragged or misaligned shapes when it applies,
 // else the skinny kernels up to kSkinnyMaxM rows and the GEMM above.
 hipError_t run_auto(const int8_t* dA, const uint8_t* dB, int32_t* dC, int M, int K, int N, Ctx& c,
@@ -920,13 +937,49 @@ hipError_t run_auto(const int8_t* dA, const uint8_t* dB, int32_t* dC, int M, int
     const hipStream_t st = c.st;
     (void)st;
     const bool pad_off = ternix_hip::debug_get(ternix_hip::DBG_RAGGED_PAD) == 0;  // tests: generic kernels
-    if (!pad_off && needs_padding(dA, dB, K, N, M <= skinny_max)) {
-        // up to 32 rows, int32 output: the whole-line GEMV reads the ragged operands as they are, one launch
+    const bool pad = needs_padding(dA, dB, K, N, M <= skinny_max);
+    // (a forced GEMV: tests and measurements of that kernel)
+    const bool forced = ternix_hip::debug_get(ternix_hip::DBG_LINE) >= 0 || ternix_hip::debug_get(ternix_hip::DBG_LINE, 3) >= 0 ||
+                        ternix_hip::debug_get(ternix_hip::DBG_SKINNY_WAVE) >= 0 || ternix_hip::debug_get(ternix_hip::DBG_SKINNY_DMA) >= 0 ||
+                        ternix_hip::debug_get(ternix_hip::DBG_M1_ATOMIC) >= 0 || ternix_hip::debug_get(ternix_hip::DBG_M1_ATOMIC, 1) >= 0 ||
+                        ternix_hip::debug_get(ternix_hip::DBG_SELF_ZERO) >= 0 || ternix_hip::debug_get(ternix_hip::DBG_WAVE_LAST) >= 0 ||
+                        ternix_hip::debug_get(ternix_hip::DBG_WAVE_SW) >= 0 || ternix_hip::debug_get(ternix_hip::DBG_DEEP) >= 0 || pad_off;
+    if (M <= skinny_max && K > 0 && K <= 65536 && !forced) {
+        const double mb = (double)K * (double)N / 4e6, mn = (double)M * (double)N * 1e-6;
+        // Rows of whole 16-byte chunks go to the GEMM unpadded; where the GEMVs would need the padded copy
+        // (N/4 % 64 != 0 or K % 64 != 0) that is their alternative above 16 rows (below, the whole-line GEMV reads
+        // them in place).  Only about as far as the estimates were fitted.
+        if (M >= 4 && K >= 256 && K <= 16384 && mb <= 32.0 && !needs_padding(dA, dB, K, N, false)) {
+            double other;
+            if (pad && M > 16) other = 1e9;
+            else if (os.Y == nullptr) other = few_rows_gemv_us(M, K, mb, mn);
+            else other = few_rows_float_us(M, K, mb, mn);
+            if (few_rows_gemm_us(K, mb) < 0.95 * other) return run_gemm(dA, dB, dC, M, K, N, c, os);
+        }
+        // Ragged operands with a float output: the int32 sums into dC (in place where dC is Y) by the whole-line GEMV
+        // and a dequantising launch, against the padded copy and a GEMV (on MI355X, warm, us: 1x659x5360 6.9 -> 5.9,
+        // 8x1000x3076 7.9 -> 7.8, 1x5056x1360 13.8 -> 5.8, 16x5056x1360 16.1 -> 10.4, 4x11204x7908 25.8 -> 18.3; 12x659x5360 7.6
+        // against 8.6, so up to 8 rows, 16 from K = 1024).  Aligned operands keep the GEMVs' own epilogues: alone the
+        // two launches are up to 12 % faster from 4 rows (16x4096x4096 9.0 -> 7.9), but with several streams at work, where
+        // launches count, slower (eight quantised layers of 8x4096x4096 34.3 against 38.7 us).
+        const bool sums = pad && (M <= 8 || (M <= 16 && K >= 1024));
+        if (os.Y != nullptr && dC != nullptr && reinterpret_cast<uintptr_t>(dC) % 16 == 0 && sums) {
+            const hipError_t e = run_auto(dA, dB, dC, M, K, N, c, ternix_hip::OutScale{}, skinny_max);
+            return e != hipSuccess ? e : TX_LAUNCH(c, ternix_hip::launch_dequant(dC, os, M, N, c.st));
+        }
+    }
+    if (!pad_off && pad) {
+        // up to 32 rows, int32 output: the whole-line GEMV reads the ragged operands as they are, one launch.
+        // 17-32 rows with a long K: the GEMM on the padded copy for float outputs (on MI355X, warm, against the GEMVs
+        // there: 24x5056x1360 19.1 -> 12.5 us, 32x11204x7908 32.8 -> 23.8; 24x1000x3076 8.1 against 9.0), and in place of the
+        // whole-line GEMV too from 16 MB of weights (32x11204x7908 38.8 -> 23; 32x3000x12000 15.7 against 16.6).
+        const bool rows = M > 16 && K > 2048 && !forced;
+        const bool heavy = rows && (long)K * (long)(N / 4) >= (16L << 20);
         hipError_t e = hipSuccess;
-        if (M <= skinny_max && os.Y == nullptr &&
+        if (M <= skinny_max && os.Y == nullptr && !heavy &&
             run_line_gemv(dA, dB, dC, M, K, N, c, &e, ternix_hip::OutScale{}, ternix_hip::ActQuant{}, 0, true))
             return e;
-        e = run_padded(dA, dB, dC, M, K, N, c, os, M <= skinny_max);
+        e = run_padded(dA, dB, dC, M, K, N, c, os, M <= skinny_max && !(rows && (heavy || os.Y != nullptr)));
         if (e != hipErrorNotSupported) return e;
     }
     if (M > skinny_max && M <= 64 && os.Y == nullptr && K % 64 == 0) {  // 33..64 rows: the atomic wave plan if it applies
@@ -1324,14 +1377,14 @@ int ternix_hip_ffn_forward(float* dY, const float* dX, const float* dNormWeight,
     float* amax = reinterpret_cast<float*>(ws + l.amax);
     hipStream_t st = static_cast<hipStream_t>(stream);
     const int m = (int)M, hd = (int)H, f = (int)F;
-    // Decode shapes: the RMSNorm + quantisation of x and the requantisation of h run inside the two
-    // skinny GEMVs (fused activation prologue, bit-identical to the standalone kernels).  Up to 4 rows
-    // with M x H <= 8192 that is two launches of the whole-line GEMV, each dequantising (and, for
-    // gate/up, applying SwiGLU) in its last-arriving split, the down launch quantising h with the
-    // gate/up launch's per-strip maxima (measured on MI355X, cold weights, 1 x 2560 x 6912: 20.2 ->
-    // 13.2 us per block); otherwise the other skinny kernels with their reduce or dequantisation
-    // launches.  Larger M: the four separate launches.
-    if (m <= kSkinnyMaxM && F > 0) {
+    // Decode shapes: up to 4 rows with M x H <= 8192 the RMSNorm + quantisation of x and the requantisation of h run
+    // inside two launches of the whole-line GEMV (bit-identical to the standalone kernels), each dequantising
+    // (and, for gate/up, applying SwiGLU) in its last-arriving split, the down launch quantising h with the
+    // gate/up launch's per-strip maxima (measured on MI355X, cold weights, 1 x 2560 x 6912: 20.2 -> 13.2 us per
+    // block).  Otherwise the four separate launches: the register-staged GEMVs with the same prologues, which took
+    // some of these shapes before, quantise every row in every workgroup (on MI355X, warm, us: 16 x 768 x 768 49.3 ->
+    // 15.1, 15 x 1536 x 2560 54.5 -> 19.6, 7 x 6144 x 512 44.0 -> 18.5, 4 x 3328 x 1280 21.0 -> 17.6).
+    if (m <= 4 && F > 0) {
         ternix_hip::OutScale os1;
         os1.Y = h;
         os1.rs = rs1;
@@ -1358,13 +1411,6 @@ int ternix_hip_ffn_forward(float* dY, const float* dX, const float* dNormWeight,
         hipError_t e = hipSuccess;
         if (ffn_line(dWgu, dWd, dY, scratch, amax, m, hd, f, os1, aq1, os2, rs2, ctx_of(st), 0, &e, &down_done)) {
             if (e != hipSuccess || down_done) return (int)e;
-            return (int)run_skinny(nullptr, dWd, reinterpret_cast<int32_t*>(dY), m, f, hd, ctx_of(st), os2, aq2);
-        }
-        const SkinnyPlan p1 = plan_skinny(m, hd, 2 * f), p2 = plan_skinny(m, f, hd);
-        if (ternix_hip::skinny_short_ok(dWgu, m, hd, 2 * f, p1.sps, p1.splits) &&
-            ternix_hip::skinny_short_ok(dWd, m, f, hd, p2.sps, p2.splits)) {
-            hipError_t e = run_skinny(nullptr, dWgu, scratch, m, hd, 2 * f, ctx_of(st), os1, aq1);
-            if (e != hipSuccess) return (int)e;
             return (int)run_skinny(nullptr, dWd, reinterpret_cast<int32_t*>(dY), m, f, hd, ctx_of(st), os2, aq2);
         }
     }
