@@ -148,7 +148,7 @@ int ternix_hip_mul_mat_ternary_noalloc(const int8_t* dA, const uint8_t* dB, int3
 size_t ternix_hip_noalloc_scratch_bytes(void);
 
 /* Frees the library-owned workspace of (current device, stream) after synchronising
- * the stream.  The caller guarantees that no hipGraph captured on that stream with
+ * the stream (NULL: the host-pointer calls' buffer too).  The caller guarantees that no hipGraph captured on that stream with
  * library calls runs again afterwards (it would reference the freed buffers).  The next
  * call on the stream allocates afresh.  Returns 0 or the hipStreamSynchronize error. */
 int ternix_hip_release_stream(void* stream);
@@ -169,9 +169,11 @@ enum ternix_hip_variant {
     TERNIX_HIP_TILED = 4
 };
 
-/* Synchronous host-pointer convenience wrapper: allocates device buffers,
- * copies A and B in, runs `variant` on the default stream, synchronises,
- * copies C out and frees every buffer on every path.
+/* Synchronous host-pointer convenience wrapper: copies A and B into a device
+ * buffer, runs `variant` on the default stream and copies C out when it is done.
+ * Calls of up to 64 MiB in all use one buffer per device that the library keeps
+ * (ternix_hip_release_stream(NULL) frees it); larger calls, and calls while
+ * another thread is inside one, allocate their own and free it on every path.
  * Replaces mul_mat_ternary_cuda_host (reference
  * include/ternix/cuda_kernels.cuh:19-21, src/cuda_kernels.cu:142-156), whose
  * bool `tiled` maps to TERNIX_HIP_TILED / TERNIX_HIP_NAIVE. */

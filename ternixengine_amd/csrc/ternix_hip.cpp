@@ -170,6 +170,59 @@ unsigned long long* zero_tickets(hipStream_t st, size_t strips) {
     return b ? reinterpret_cast<unsigned long long*>(b + kCounterSlots) : nullptr;
 }
 
+// Device buffer of one host-pointer call.  hipMalloc and hipFree of three buffers and a device-wide wait took 40 of 245 us
+// (16 x 2560 x 6912; the rest is the pageable copies, 4.4 MB up in 144 us), so one buffer per device of up to kHostBufferMax bytes is kept between calls, until
+// ternix_hip_release_stream(NULL); a call that finds it in use (another thread) or needs more than that allocates
+// its own and frees it.
+constexpr size_t kHostBufferMax = size_t(64) << 20;
+struct HostPool {
+    std::mutex m;
+    char* ptr = nullptr;
+    size_t bytes = 0;
+};
+HostPool g_host_pool[16];
+struct HostBuffer {
+    char* ptr = nullptr;
+    HostPool* pool = nullptr;  // locked while this call uses its buffer
+    bool idle = false;         // nothing queued uses the buffer any more
+    explicit HostBuffer(size_t bytes) {
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess) return;
+        if (bytes <= kHostBufferMax && dev >= 0 && dev < 16 && g_host_pool[dev].m.try_lock()) {
+            pool = &g_host_pool[dev];
+            if (pool->bytes < bytes) {
+                if (pool->ptr) (void)hipFree(pool->ptr);
+                pool->ptr = nullptr;
+                pool->bytes = std::min(kHostBufferMax, std::max(bytes, size_t(1) << 20) * 2);
+                void* p = nullptr;
+                if (lib_malloc(&p, pool->bytes) != hipSuccess) pool->bytes = 0;
+                pool->ptr = static_cast<char*>(p);
+            }
+            ptr = pool->ptr;
+            return;
+        }
+        void* p = nullptr;
+        if (lib_malloc(&p, bytes ? bytes : 16) == hipSuccess) ptr = static_cast<char*>(p);
+    }
+    HostBuffer(const HostBuffer&) = delete;
+    HostBuffer& operator=(const HostBuffer&) = delete;
+    ~HostBuffer() {
+        if (pool) {
+            if (!idle) (void)hipStreamSynchronize(nullptr);  // a call that failed half-way
+            pool->m.unlock();
+        } else if (ptr) {
+            (void)hipFree(ptr);
+        }
+    }
+};
+void release_host_pool(int dev) {
+    if (dev < 0 || dev >= 16) return;
+    std::lock_guard<std::mutex> lock(g_host_pool[dev].m);
+    if (g_host_pool[dev].ptr) (void)hipFree(g_host_pool[dev].ptr);
+    g_host_pool[dev].ptr = nullptr;
+    g_host_pool[dev].bytes = 0;
+}
+
 // Execution context of one call: the stream, where split-K partials and padded copies live, and a
 // dry-run mode for planning queries.
 //   * library-owned workspace (default): the per-(device, stream) buffers above;
@@ -1150,6 +1203,7 @@ int ternix_hip_release_stream(void* stream) {
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return (int)e;
+    if (st == nullptr) release_host_pool(dev);
     Workspace w;
     {
         std::lock_guard<std::mutex> lock(g_ws_mutex);
@@ -1199,34 +1253,26 @@ int ternix_hip_mul_mat_ternary_host(const int8_t* A, const uint8_t* B_packed, in
     if (trivial) return (int)hipSuccess;
     const size_t a_bytes = (size_t)M * (size_t)K, b_bytes = (size_t)K * (size_t)(N / 4),
                  c_bytes = (size_t)M * (size_t)N * sizeof(int32_t);
-    int8_t* dA = nullptr;
-    uint8_t* dB = nullptr;
-    int32_t* dC = nullptr;
-    // hipMalloc of 0 bytes returns a null pointer; keep the pointers non-null for validation.
-    if ((e = lib_malloc(reinterpret_cast<void**>(&dA), a_bytes ? a_bytes : 16)) != hipSuccess) goto done;
-    if ((e = lib_malloc(reinterpret_cast<void**>(&dB), b_bytes ? b_bytes : 16)) != hipSuccess) goto done;
-    if ((e = lib_malloc(reinterpret_cast<void**>(&dC), c_bytes)) != hipSuccess) goto done;
-    if (a_bytes && (e = hipMemcpy(dA, A, a_bytes, hipMemcpyHostToDevice)) != hipSuccess) goto done;
-    if (b_bytes && (e = hipMemcpy(dB, B_packed, b_bytes, hipMemcpyHostToDevice)) != hipSuccess) goto done;
-    {
-        int s;
-        switch (variant) {
-            case TERNIX_HIP_NAIVE: s = ternix_hip_mul_mat_ternary_naive(dA, dB, dC, M, K, N, nullptr); break;
-            case TERNIX_HIP_GEMV: s = ternix_hip_mul_mat_ternary_gemv(dA, dB, dC, M, K, N, nullptr); break;
-            case TERNIX_HIP_GEMM: s = ternix_hip_mul_mat_ternary_gemm(dA, dB, dC, M, K, N, nullptr); break;
-            case TERNIX_HIP_TILED: s = ternix_hip_mul_mat_ternary_tiled(dA, dB, dC, M, K, N, nullptr); break;
-            default: s = ternix_hip_mul_mat_ternary(dA, dB, dC, M, K, N, nullptr); break;
-        }
-        e = static_cast<hipError_t>(s);
+    auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
+    HostBuffer buf(up(a_bytes) + up(b_bytes) + c_bytes);
+    if (buf.ptr == nullptr) return (int)hipErrorOutOfMemory;
+    int8_t* dA = reinterpret_cast<int8_t*>(buf.ptr);
+    uint8_t* dB = reinterpret_cast<uint8_t*>(buf.ptr + up(a_bytes));
+    int32_t* dC = reinterpret_cast<int32_t*>(buf.ptr + up(a_bytes) + up(b_bytes));
+    if (a_bytes && (e = hipMemcpy(dA, A, a_bytes, hipMemcpyHostToDevice)) != hipSuccess) return (int)e;
+    if (b_bytes && (e = hipMemcpy(dB, B_packed, b_bytes, hipMemcpyHostToDevice)) != hipSuccess) return (int)e;
+    int s;
+    switch (variant) {
+        case TERNIX_HIP_NAIVE: s = ternix_hip_mul_mat_ternary_naive(dA, dB, dC, M, K, N, nullptr); break;
+        case TERNIX_HIP_GEMV: s = ternix_hip_mul_mat_ternary_gemv(dA, dB, dC, M, K, N, nullptr); break;
+        case TERNIX_HIP_GEMM: s = ternix_hip_mul_mat_ternary_gemm(dA, dB, dC, M, K, N, nullptr); break;
+        case TERNIX_HIP_TILED: s = ternix_hip_mul_mat_ternary_tiled(dA, dB, dC, M, K, N, nullptr); break;
+        default: s = ternix_hip_mul_mat_ternary(dA, dB, dC, M, K, N, nullptr); break;
     }
-    if (e != hipSuccess) goto done;
-    if ((e = hipDeviceSynchronize()) != hipSuccess) goto done;
+    if (s != 0) return s;
+    // (the copy runs after the kernel on the default stream, returns when it is done, and reports its error)
     e = hipMemcpy(C, dC, c_bytes, hipMemcpyDeviceToHost);
-done:
-    // Free on every path; a free failure never masks the first error.
-    if (dA) (void)hipFree(dA);
-    if (dB) (void)hipFree(dB);
-    if (dC) (void)hipFree(dC);
+    buf.idle = e == hipSuccess;
     return (int)e;
 }
 
