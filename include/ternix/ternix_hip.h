@@ -210,7 +210,8 @@ int ternix_hip_device_count(void);
  *   "gemm_generic" v0   1: the generic GEMM for every GEMM call
  *   "gemm_splits" v0    GEMM split-K count forced
  *   "gemm_bm" v0,v1     v0 64 / 128: GEMM tile height forced (256: as 128); v1 0-6: tile shape
- *                       of the 32x32x32 MFMA GEMM forced
+ *                       of the 32x32x32 MFMA GEMM forced (7, 8: tiles 0 and 1 reading
+ *                       ragged operands in place)
  *   "gemm_gm" v0        row tiles per group in the tile order of the GEMMs
  *   "deep" v0..3        0: no whole-K deep GEMV; else force (strip bytes, waves
  *                       per workgroup, ring slots, splits)

@@ -483,6 +483,11 @@ void gemm_pipe16_kernel(const int8_t* __restrict__ A, const uint8_t* __restrict_
 // k-step).  DMAs in one burst after the barrier cost 6 % (1024x6912x2560 24.0 -> 22.0 us).
 // us before -> after, L2-warm weights: 128x4096x4096 19.3 -> 9.5, 256x4096x11008 20.7 -> 16.7, 1024x6912x2560 31.4 ->
 // 22.1, 1024x2560x13824 41 -> 34.5, 2048x4096x14336 126 -> 111 (the card at its slowest; 103 -> 98 otherwise).
+// RG: ragged operands (any K >= BK, NB >= BNB, any addresses) read in place.  Every 16-byte chunk lies inside its row,
+// since the last stage ends at k_end and the last column tile at NB (both overlap their neighbour; columns done
+// twice store the same values), so chunks go through registers with one unaligned load each, no edge cases, and
+// from there to the same LDS slots: two stages in LDS, the next two in registers.  Rows of W already done are
+// zeroed on the way instead of masked.
 // LDS layouts (no bank conflicts): A chunk c of row r at c ^ ((r/2) % 8) for 128-byte rows, c ^ (r % 16) for
 // 256-byte ones; W's 32-byte column pairs p of row r at p ^ f(r), f the row bits that make 8 rows of one pair
 // cover all 64 banks.  W fragments come from ds_read_b64_tr_b8 (see below): 16-lane groups 0-1 take the two
@@ -519,7 +524,7 @@ struct WideFrag {
     uint64_t lo, hi;
 };
 
-template <int WGM, int WGN, int WGK, int MT, int BK, int NS, bool TILED, int GM>
+template <int WGM, int WGN, int WGK, int MT, int BK, int NS, bool TILED, int GM, bool RG>
 __global__ __launch_bounds__(64 * WGM * WGN * WGK) __attribute__((amdgpu_waves_per_eu(2)))
 void gemm_pipe_kernel(const int8_t* __restrict__ A, const uint8_t* __restrict__ B, int32_t* __restrict__ C, int M,
                       int K, int N, int n_out, int tiles_n, int k_begin, int k_end, int accumulate, int vec_store,
@@ -568,7 +573,7 @@ void gemm_pipe_kernel(const int8_t* __restrict__ A, const uint8_t* __restrict__ 
         tn = local / gm;
     }
     const int row0 = tm * BM;
-    const int bc0 = tn * BNB;
+    const int bc0 = RG ? min(tn * BNB, NB - BNB) : tn * BNB;
     // Stages of BK k-rows; the last one ends at k_end, so where BK does not divide the range it starts inside
     // the stage before, and the rows that one has done are masked out of its weights.
     const int klen = k_end - k_begin;
@@ -589,7 +594,8 @@ void gemm_pipe_kernel(const int8_t* __restrict__ A, const uint8_t* __restrict__ 
         const int slot = (p * NWV + wave) * 64 + lane;
         const int r = slot / CW, pos = slot % CW;
         const int c = min((bc0 >> 4) + (pos ^ gw_swz_w<BNB>(r)), (NB >> 4) - 1);  // columns past N: never stored
-        w_off[p] = TILED ? tile64_offset(c, r, K >> 6) : (uint32_t)r * (uint32_t)NB + (uint32_t)(c * 16);
+        if (RG) w_off[p] = (uint32_t)r * (uint32_t)NB + (uint32_t)(bc0 + (pos ^ gw_swz_w<BNB>(r)) * 16);
+        else w_off[p] = TILED ? tile64_offset(c, r, K >> 6) : (uint32_t)r * (uint32_t)NB + (uint32_t)(c * 16);
     }
     // DMA instruction d of stage st (A's NA, then W's NW) into the stage buffer at byte `off`.
     // (Stages past the last one repeat it: the load count per stage stays static, and a branch around the
@@ -603,6 +609,21 @@ void gemm_pipe_kernel(const int8_t* __restrict__ A, const uint8_t* __restrict__ 
             const uint8_t* wbase = TILED ? B + (size_t)(k0 >> 6) * 1024 : B + (size_t)k0 * (size_t)NB;
             lds_dma16(wbase + w_off[p < 0 ? 0 : p], smem + off + A_STAGE + (p * NWV + wave) * 1024);
         }
+    };
+
+    // Ragged operands (RG): chunk d of stage st through a register, and from there into the stage buffer.
+    auto gload = [&](int st, int d) -> v4i {
+        const int k0 = k_begin + min(st * BK, klen - BK);
+        const void* src = d < NA ? (const void*)(A + k0 + a_off[d < NA ? d : 0])
+                                 : (const void*)(B + (size_t)k0 * (size_t)NB + w_off[d < NA ? 0 : d - NA]);
+        v4i v;
+        __builtin_memcpy(&v, src, 16);  // any alignment
+        return v;
+    };
+    auto swrite = [&](v4i v, int st, int off, int d) {
+        const int slot = ((d < NA ? d : d - NA) * NWV + wave) * 64 + lane;
+        if (d >= NA && st == nst - 1 && slot / CW < done) v = v4i{0, 0, 0, 0};  // a k-row the stage before has done
+        lds_write_b128_asm(lds_u32(smem) + (uint32_t)(off + (d < NA ? 0 : A_STAGE) + slot * 16), v);
     };
 
     uint32_t a_lane[KS];
@@ -645,7 +666,7 @@ void gemm_pipe_kernel(const int8_t* __restrict__ A, const uint8_t* __restrict__ 
     // Field mask of each k-step: all fields, or none in the last stage's steps that are already done (a lane
     // holds 16 consecutive k-rows of a step, and every k-range is a multiple of 16 rows).
     auto field_mask = [&](bool last, int kk) -> uint32_t {
-        return last && (wk * KS + kk) * 32 + half * 16 < done ? 0u : 0xC0C0C0C0u;
+        return !RG && last && (wk * KS + kk) * 32 + half * 16 < done ? 0u : 0xC0C0C0C0u;
     };
     uint32_t mask[KS];
 #pragma unroll
@@ -661,11 +682,31 @@ void gemm_pipe_kernel(const int8_t* __restrict__ A, const uint8_t* __restrict__ 
     constexpr int R = 2 + MT;       // LDS reads per k-step
 
     WideFrag<MT> f0, f1;
+    v4i ga[RG ? D : 1], gb[RG ? D : 1];  // RG: the chunks of stages st + 2 (even st: ga) and st + 3
+    if constexpr (RG) {
+        static_assert(NS == 2 && !TILED, "two stage buffers, two stages in registers");
 #pragma unroll
-    for (int p = 0; p < NS; ++p)
+        for (int d = 0; d < D; ++d) ga[d] = gload(0, d);
 #pragma unroll
-        for (int d = 0; d < D; ++d) issue(p, p * STAGE, d);
-    TX_VMCNT((NS - 1) * D);
+        for (int d = 0; d < D; ++d) gb[d] = gload(1, d);
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            swrite(ga[d], 0, 0, d);
+            ga[d] = gload(2, d);
+        }
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            swrite(gb[d], 1, STAGE, d);
+            gb[d] = gload(3, d);
+        }
+        TX_LGKMCNT0();
+    } else {
+#pragma unroll
+        for (int p = 0; p < NS; ++p)
+#pragma unroll
+            for (int d = 0; d < D; ++d) issue(p, p * STAGE, d);
+        TX_VMCNT((NS - 1) * D);
+    }
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -677,12 +718,12 @@ void gemm_pipe_kernel(const int8_t* __restrict__ A, const uint8_t* __restrict__ 
 
     // One 32-row k-step: SLOTS MFMAs, each followed by a share of the next field's decode, of the next
     // k-step's LDS reads (first half) and, in a stage's last k-step, of the DMAs of stage st + NS.
-    auto step = [&](auto kc, WideFrag<MT>& cur, WideFrag<MT>& nxt, int st, uint32_t off, uint32_t noff) {
+    auto step = [&](auto kc, WideFrag<MT>& cur, WideFrag<MT>& nxt, int st, uint32_t off, uint32_t noff, v4i* g) {
         constexpr int KK = decltype(kc)::value;
         constexpr bool LAST = KK + 1 == KS;
         if constexpr (LAST) {
             // stage st + 1 has landed (the NS - 2 later ones may not)
-            TX_VMCNT((NS - 2) * D);
+            if constexpr (!RG) TX_VMCNT((NS - 2) * D);
             __builtin_amdgcn_s_barrier();  // ... everywhere, and every wave is done reading stage st
         }
         if (LAST && done > 0 && st + 2 == nst) {
@@ -708,7 +749,14 @@ void gemm_pipe_kernel(const int8_t* __restrict__ A, const uint8_t* __restrict__ 
             if constexpr (LAST) {
 #pragma unroll
                 for (int d = 0; d < D; ++d)
-                    if (d * SLOTS / D == s) issue(st + NS, (int)off, d);
+                    if (d * SLOTS / D == s) {
+                        if constexpr (RG) {
+                            swrite(g[d], st + 2, (int)off, d);
+                            g[d] = gload(st + 4, d);
+                        } else {
+                            issue(st + NS, (int)off, d);
+                        }
+                    }
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -716,16 +764,26 @@ void gemm_pipe_kernel(const int8_t* __restrict__ A, const uint8_t* __restrict__ 
         if (LAST && done > 0 && st + 2 == nst) mask[KS - 1] = field_mask(true, KS - 1);
         __builtin_amdgcn_sched_barrier(0);
     };
-    uint32_t off = 0;
-    for (int st = 0; st < nst; ++st) {
-        const uint32_t noff = off + STAGE == (uint32_t)(NS * STAGE) ? 0u : off + STAGE;
-        step(Int<0>{}, f0, f1, st, off, noff);
-        step(Int<1>{}, f1, f0, st, off, noff);
+    auto stage = [&](int st, uint32_t off, uint32_t noff, v4i* g) {
+        step(Int<0>{}, f0, f1, st, off, noff, g);
+        step(Int<1>{}, f1, f0, st, off, noff, g);
         if constexpr (KS == 4) {
-            step(Int<2>{}, f0, f1, st, off, noff);
-            step(Int<3>{}, f1, f0, st, off, noff);
+            step(Int<2>{}, f0, f1, st, off, noff, g);
+            step(Int<3>{}, f1, f0, st, off, noff, g);
         }
-        off = noff;
+    };
+    if constexpr (RG) {
+        for (int st = 0; st < nst; st += 2) {
+            stage(st, 0, STAGE, ga);
+            if (st + 1 < nst) stage(st + 1, STAGE, 0, gb);
+        }
+    } else {
+        uint32_t off = 0;
+        for (int st = 0; st < nst; ++st) {
+            const uint32_t noff = off + STAGE == (uint32_t)(NS * STAGE) ? 0u : off + STAGE;
+            stage(st, off, noff, ga);
+            off = noff;
+        }
     }
     // The float epilogue's row scales, all in flight at once (loaded one by one between the stores they cost a
     // memory latency per row: dequantising 1024x2560x13824 38.3 us against 34 for int32).
@@ -816,19 +874,22 @@ constexpr WideTile kWide[kWideTiles] = {
 // The 64 x 256 tiles of gemm_pipe16_kernel, on the same scale.
 constexpr WideTile kPipe64Cost = {64, 64, 128, 2, 1.08f, 1.76f, 0.001f, 4.75f, 0.225f, 0.732f};
 
-template <int WGM, int WGN, int WGK, int MT, int BK, int NS, int GM>
+template <int WGM, int WGN, int WGK, int MT, int BK, int NS, int GM, bool RG = false>
 hipError_t launch_wide(const int8_t* A, const uint8_t* B, int32_t* C, int M, int K, int N, int n_out, int kb, int ke,
                        int acc, int vs, hipStream_t st, const OutScale& os, int splits, int k_split, int tiled,
                        int gm_env) {
     constexpr int BM = 32 * MT * WGM, BNB = 32 * WGN;
     const int tiles_n = (N / 4 + BNB - 1) / BNB;
     const dim3 grid((unsigned)(((M + BM - 1) / BM) * tiles_n), splits), block(64 * WGM * WGN * WGK);
-    if (tiled)
-        hipLaunchKernelGGL((gemm_pipe_kernel<WGM, WGN, WGK, MT, BK, NS, true, GM>), grid, block, 0, st, A, B, C, M, K, N,
-                           n_out, tiles_n, kb, ke, acc, vs, k_split, os, gm_env);
-    else
-        hipLaunchKernelGGL((gemm_pipe_kernel<WGM, WGN, WGK, MT, BK, NS, false, GM>), grid, block, 0, st, A, B, C, M, K, N,
-                           n_out, tiles_n, kb, ke, acc, vs, k_split, os, gm_env);
+    if constexpr (!RG) {
+        if (tiled) {
+            hipLaunchKernelGGL((gemm_pipe_kernel<WGM, WGN, WGK, MT, BK, NS, true, GM, false>), grid, block, 0, st, A, B, C, M, K,
+                               N, n_out, tiles_n, kb, ke, acc, vs, k_split, os, gm_env);
+            return hipGetLastError();
+        }
+    }
+    hipLaunchKernelGGL((gemm_pipe_kernel<WGM, WGN, WGK, MT, BK, NS, false, GM, RG>), grid, block, 0, st, A, B, C, M, K, N,
+                       n_out, tiles_n, kb, ke, acc, vs, k_split, os, gm_env);
     return hipGetLastError();
 }
 
@@ -928,6 +989,12 @@ void split_k(int K, long splits, int least, GemmPlan* p) {
     p->k_split = 0;
 }
 
+// Sizes the ragged tiles take: a whole stage, a whole tile of columns, 32-bit offsets.
+bool ragged_ok(int M, int K, int N) {
+    return M > 0 && K >= 256 && N / 4 >= 64 && (size_t)M * (size_t)K < ((size_t)1 << 32) &&
+           (size_t)256 * (size_t)(N / 4) < ((size_t)1 << 32);
+}
+
 // The split count of the row-tile plan (gemm_split_rows): one workgroup per CU, at most 16 splits of >= 256 rows.
 int row_tile_splits(int M, int K, int N, int bm, int col_tiles) {
     // K <= 4096: the reduce launch and the partial sums cost more than the idle CUs (measured on
@@ -958,6 +1025,12 @@ GemmPlan gemm_plan(const int8_t* A, const uint8_t* B, int M, int K, int N, int t
     }
     const int splits_env = debug_get(DBG_GEMM_SPLITS);  // tests
     auto forced = [&](long s) { return splits_env > 0 ? (long)splits_env : s; };
+    const int tile_rg = debug_get(DBG_GEMM_BM, 1) - kWideTiles;  // tests and measurements
+    if (tile_rg >= 0 && tile_rg < kRaggedTiles && !tiled && ragged_ok(M, K, N)) {
+        p.choice = (GemmChoice)((int)GemmChoice::Ragged0 + tile_rg);
+        if (may_split) split_k(K, forced(1), 256, &p);
+        return p;
+    }
     if (!pipe16 && !wide) {
         if (may_split) split_k(K, forced(row_tile_splits(M, K, N, gemm_split_rows(M, K, N), (NB + 63) / 64)), 64, &p);
         return p;  // Generic
@@ -1031,6 +1104,37 @@ GemmPlan gemm_plan(const int8_t* A, const uint8_t* B, int M, int K, int N, int t
     return p;
 }
 
+// Ragged tiles, where one round of workgroups holds the whole output: the padded copy (6.6 us for 129x8191x2052) costs
+// more than their unaligned loads.  Over more rounds the copy is read often enough to pay (400x1001x5004, 260 tiles,
+// 16.8 against 14.4 us).  On MI355X, warm, us, padded copy / in place: 129x8191x2052 18.6 / 15.0, 65x4093x4100 15.1 / 12.0,
+// 33x12001x3004 21.0 / 14.6, 513x8481x804 22.9 / 17.6, 257x1001x5004 12.0 / 9.7, 33x1001x516 8.4 / 8.8.
+GemmPlan gemm_ragged_plan(int M, int K, int N, bool may_split) {
+    // Fitted to 780 timings of 108 ragged shapes (rms error 9 %), as kWide.
+    static constexpr WideTile cost[kRaggedTiles] = {
+        {32, 32, 256, 2, 0.631f, 1.40f, 2.43f, 4.22f, 1.0f, 0.809f},
+        {32, 64, 256, 2, 0.745f, 1.93f, 0.0f, 6.83f, 0.915f, 0.707f},
+    };
+    GemmPlan p;
+    p.choice = GemmChoice::Invalid;
+    const bool forced = debug_get(DBG_GEMM_BM) > 0 || debug_get(DBG_GEMM_BM, 1) >= 0 || debug_get(DBG_GEMM_GENERIC) == 1 ||
+                        debug_get(DBG_GEMM_NARROW) >= 0 || debug_get(DBG_GEMM_SPLITS) > 0;  // tests of the other kernels
+    if (!ragged_ok(M, K, N) || forced) return p;
+    const long cus = device_cu_count();
+    double best = 1e30;
+    for (int i = 0; i < kRaggedTiles; ++i) {
+        const long tiles = (long)((M + cost[i].rows - 1) / cost[i].rows) * (long)((N / 4 + cost[i].bnb - 1) / cost[i].bnb);
+        for (const long s : {1L, 2L, 3L, 4L, 6L, 8L, 12L, 16L}) {
+            if (tiles * s > cus || (s > 1 && (!may_split || K / s < 384))) break;
+            const double t = wide_cost(cost[i], M, N, (K + s - 1) / s, s);
+            if (t >= best) continue;
+            best = t;
+            p.choice = (GemmChoice)((int)GemmChoice::Ragged0 + i);
+            split_k(K, s, 256, &p);
+        }
+    }
+    return p;
+}
+
 const char* gemm_choice_name(GemmChoice c) {
     switch (c) {
         case GemmChoice::Narrow64: return "gemm_pipe_kernel<64 rows x 64 cols, 4 waves, 16x16x64>";
@@ -1042,6 +1146,8 @@ const char* gemm_choice_name(GemmChoice c) {
         case GemmChoice::Wide4: return "gemm_pipe_kernel<64 rows x 512 cols, 4 waves>";
         case GemmChoice::Wide5: return "gemm_pipe_kernel<64 rows x 256 cols, K over 2 of 4 waves>";
         case GemmChoice::Wide6: return "gemm_pipe_kernel<128 rows x 256 cols, K over 2 of 8 waves>";
+        case GemmChoice::Ragged0: return "gemm_pipe_kernel ragged<32 rows x 128 cols, K over 4 waves>";
+        case GemmChoice::Ragged1: return "gemm_pipe_kernel ragged<32 rows x 256 cols, K over 4 of 8 waves>";
         case GemmChoice::Generic: return "gemm_kernel<128 rows x 256 cols, register-staged>";
         default: return "invalid";
     }
@@ -1092,7 +1198,9 @@ hipError_t launch_gemm(const GemmPlan& p, const int8_t* A, const uint8_t* B, int
         case GemmChoice::Wide3: return TX_WIDE(1, 4, 2, 2, 128, 4, 8);
         case GemmChoice::Wide4: return TX_WIDE(1, 4, 1, 2, 128, 3, 8);
         case GemmChoice::Wide5: return TX_WIDE(1, 2, 2, 2, 128, 3, 8);
-        default: return TX_WIDE(2, 2, 2, 2, 128, 4, 4);
+        case GemmChoice::Wide6: return TX_WIDE(2, 2, 2, 2, 128, 4, 4);
+        case GemmChoice::Ragged0: return TX_WIDE(1, 1, 4, 1, 256, 2, 8, true);
+        default: return TX_WIDE(1, 2, 4, 1, 256, 2, 8, true);
     }
 #undef TX_WIDE
 }

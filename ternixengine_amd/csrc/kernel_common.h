@@ -238,6 +238,9 @@ __device__ __forceinline__ void lds_write_b8_asm(uint32_t addr, uint32_t v) {
 __device__ __forceinline__ void lds_write_b32_asm(uint32_t addr, uint32_t v) {
     __asm__ volatile("ds_write_b32 %0, %1" : : "v"(addr), "v"(v) : "memory");
 }
+__device__ __forceinline__ void lds_write_b128_asm(uint32_t addr, v4i v) {
+    __asm__ volatile("ds_write_b128 %0, %1" : : "v"(addr), "v"(v) : "memory");
+}
 __device__ __forceinline__ uint32_t lds_u32(const void* p) {
     return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p;
 }

@@ -38,7 +38,8 @@ enum DebugKey : int {
     DBG_GEMM_NARROW,     // [0] 0 / 1: 64 x 64 GEMM tiles for M <= 64 off / forced
     DBG_GEMM_GENERIC,    // [0] == 1: the generic (register-staged) GEMM for every GEMM call
     DBG_GEMM_SPLITS,     // [0] GEMM split-K count forced
-    DBG_GEMM_BM,         // [0] 64 / 128: GEMM tile height forced (256: as 128); [1] gemm_pipe_kernel tile forced (0-6)
+    DBG_GEMM_BM,         // [0] 64 / 128: GEMM tile height forced (256: as 128); [1] gemm_pipe_kernel tile forced (0-6; 7, 8:
+                         //     tiles 0 and 1 reading ragged operands)
     DBG_DEEP,            // [0] == 0: no whole-K deep GEMV; else (sw, nw, nsw, splits) forced
     DBG_SK_ORDER,        // [0] 1: release/acquire (agent scope) for the in-launch split sums
     DBG_M1_ATOMIC,       // [0] 0: no zero-fill + atomic split plan for M = 1 GEMVs; [1] / [2] largest M of
@@ -154,9 +155,10 @@ hipError_t launch_skinny_wave(const int8_t* A, const uint8_t* B, int32_t* C, int
 bool gemm_narrow_wanted(int M, int K, int N, int tiled = 0);
 // Tile height (64 or 128 rows) launch_gemm uses for this shape when K is split.
 int gemm_split_rows(int M, int K, int N);
-// The GEMM kernel of a call and its K split.  Wide0 ..: gemm_pipe_kernel's tile shapes.
-enum class GemmChoice { Invalid, Generic, Narrow64, Pipe64, Wide0, Wide1, Wide2, Wide3, Wide4, Wide5, Wide6 };
-constexpr int kWideTiles = 7;
+// The GEMM kernel of a call and its K split.  Wide0 ..: gemm_pipe_kernel's tile shapes; Ragged0, Ragged1: the first two
+// of them reading ragged operands in place.
+enum class GemmChoice { Invalid, Generic, Narrow64, Pipe64, Wide0, Wide1, Wide2, Wide3, Wide4, Wide5, Wide6, Ragged0, Ragged1 };
+constexpr int kWideTiles = 7, kRaggedTiles = 2;
 struct GemmPlan {
     GemmChoice choice = GemmChoice::Generic;
     int splits = 1, k_split = 0;
@@ -165,6 +167,8 @@ struct GemmPlan {
 // fewer columns than N, which only gemm_pipe_kernel stores (the others through slabs of N columns).
 GemmPlan gemm_plan(const int8_t* A, const uint8_t* B, int M, int K, int N, int tiled, bool may_split,
                    bool padded = false);
+// Ragged operands (any K >= 256, N / 4 >= 64, any addresses) in place, or Invalid where the padded copy is better.
+GemmPlan gemm_ragged_plan(int M, int K, int N, bool may_split);
 const char* gemm_choice_name(GemmChoice c);
 // LDS-tiled MFMA GEMM over k-rows [k_begin, k_end); accumulate != 0 adds into C instead of storing.
 // With os.Y set the tile epilogue writes the dequantised floats instead (accumulate must be 0).

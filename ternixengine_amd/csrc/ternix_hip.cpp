@@ -838,15 +838,16 @@ hipError_t run_skinny(const int8_t* dA, const uint8_t* dB, int32_t* dC, int M, i
 }
 
 // GEMMs: gemm_plan picks the kernel and its K split (few output tiles against a long K); partial tiles of a
-// split go through the same workspace and reduce launch as the skinny path.
+// split go through the same workspace and reduce launch as the skinny path.  ragged: the operands as they are,
+// where gemm_ragged_plan has a plan.
 hipError_t run_gemm(const int8_t* dA, const uint8_t* dB, int32_t* dC, int M, int K, int N, Ctx& c,
-                    const ternix_hip::OutScale& os = ternix_hip::OutScale{}, int tiled = 0) {
+                    const ternix_hip::OutScale& os = ternix_hip::OutScale{}, int tiled = 0, bool ragged = false) {
     const hipStream_t st = c.st;
     (void)st;
     using ternix_hip::GemmChoice;
     using ternix_hip::GemmPlan;
     if (K <= ternix_hip::kMaxKPerAccumulator) {
-        GemmPlan p = ternix_hip::gemm_plan(dA, dB, M, K, N, tiled, true);
+        GemmPlan p = ragged ? ternix_hip::gemm_ragged_plan(M, K, N, true) : ternix_hip::gemm_plan(dA, dB, M, K, N, tiled, true);
         if (p.splits > 1) {
             const size_t need = (size_t)p.splits * (size_t)M * (size_t)N * sizeof(int32_t);
             int32_t* partials = need <= kWorkspaceMax ? static_cast<int32_t*>(c.get(need)) : nullptr;
@@ -857,7 +858,7 @@ hipError_t run_gemm(const int8_t* dA, const uint8_t* dB, int32_t* dC, int M, int
                 if (e != hipSuccess) return e;
                 return TX_LAUNCH(c, ternix_hip::launch_splitk_reduce(partials, dC, M, N, p.splits, os, st));
             }
-            p = ternix_hip::gemm_plan(dA, dB, M, K, N, tiled, false);
+            p = ragged ? ternix_hip::gemm_ragged_plan(M, K, N, false) : ternix_hip::gemm_plan(dA, dB, M, K, N, tiled, false);
         }
         c.note("%s", ternix_hip::gemm_choice_name(p.choice));
         return TX_LAUNCH(c, ternix_hip::launch_gemm(p, dA, dB, dC, M, K, N, 0, K, 0, st, os, tiled));
@@ -1032,7 +1033,12 @@ hipError_t run_auto(const int8_t* dA, const uint8_t* dB, int32_t* dC, int M, int
         if (M <= skinny_max && os.Y == nullptr && !heavy &&
             run_line_gemv(dA, dB, dC, M, K, N, c, &e, ternix_hip::OutScale{}, ternix_hip::ActQuant{}, 0, true))
             return e;
-        e = run_padded(dA, dB, dC, M, K, N, c, os, M <= skinny_max && !(rows && (heavy || os.Y != nullptr)));
+        const bool gemm = M > skinny_max || (rows && (heavy || os.Y != nullptr));
+        // (rows of whole chunks at odd addresses keep the copy)
+        if (gemm && (K % 16 != 0 || (N / 4) % 16 != 0) && K <= ternix_hip::kMaxKPerAccumulator &&
+            ternix_hip::gemm_ragged_plan(M, K, N, true).choice != ternix_hip::GemmChoice::Invalid)
+            return run_gemm(dA, dB, dC, M, K, N, c, os, 0, true);
+        e = run_padded(dA, dB, dC, M, K, N, c, os, !gemm);
         if (e != hipErrorNotSupported) return e;
     }
     if (M > skinny_max && M <= 64 && os.Y == nullptr && K % 64 == 0) {  // 33..64 rows: the atomic wave plan if it applies

@@ -71,6 +71,53 @@ def test_padded_copy_writes_the_real_columns(lib, oracle, shape):
     np.testing.assert_array_equal(y.view(np.float32), ref.astype(np.float32) * (rs * np.float32(0.25))[:, None])
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", [7, 8])
+@pytest.mark.parametrize("splits", [1, 3])
+def test_ragged_tiles_read_in_place(lib, oracle, tile, splits):
+    """The ragged forms: sizes and addresses off every boundary, the smallest K and N they take, last stages and
+    column tiles that overlap their neighbours, operands that end where their buffers do."""
+    rng = np.random.default_rng(tile)
+    for m, k, n, ao, wo in ((1, 256, 256, 0, 0), (31, 257, 260, 1, 3), (33, 511, 516, 2, 0), (65, 1001, 508, 3, 1),
+                            (129, 769, 1028, 0, 2), (40, 2049, 2044, 1, 1)):
+        print(f"ragged tile {tile} splits {splits} M={m} K={k} N={n} A+{ao} W+{wo}", flush=True)
+        a = rng.integers(-128, 128, size=(m, k), dtype=np.int8)
+        wp = rng.integers(0, 256, size=(k, n // 4), dtype=np.uint8)
+        ref = oracle.mm("scalar_mt", a, wp, n)
+        da = hr.DeviceBuffer.from_array(np.concatenate([np.zeros(ao, np.int8), a.reshape(-1)]))
+        dw = hr.DeviceBuffer.from_array(np.concatenate([np.zeros(wo, np.uint8), wp.reshape(-1)]))
+        dc = hr.DeviceBuffer(4 * m * n + 64)
+        assert lib.ternix_hip_debug_set(b"gemm_bm", -1, tile, -1, -1) == 0
+        assert lib.ternix_hip_debug_set(b"gemm_splits", splits, -1, -1, -1) == 0
+        dc.upload(np.full(m * n + 16, -7, np.int32))
+        assert lib.ternix_hip_mul_mat_ternary_gemm(da.value + ao, dw.value + wo, dc.value, m, k, n, None) == 0
+        hr.synchronize()
+        got = dc.download(np.int32, (m * n + 16,))
+        assert (got[:m * n].reshape(m, n) == ref).all() and (got[m * n:] == -7).all(), (m, k, n)
+
+
+@pytest.mark.gpu
+def test_ragged_plans_first_call_inside_capture(oracle):
+    """A ragged call whose plan splits K, captured on a fresh stream (no workspace: one split), then eager."""
+    lib = tx._load()
+    m, k, n = 65, 4093, 1028
+    rng = np.random.default_rng(5)
+    a, wp = rng.integers(-128, 128, size=(m, k), dtype=np.int8), rng.integers(0, 256, size=(k, n // 4), dtype=np.uint8)
+    ref = oracle.mm("scalar_mt", a, wp, n)
+    da, dw, dc, s = hr.DeviceBuffer.from_array(a), hr.DeviceBuffer.from_array(wp), hr.DeviceBuffer(4 * m * n), hr.Stream()
+
+    def call():
+        assert lib.ternix_hip_mul_mat_ternary(da.value, dw.value, dc.value, m, k, n, s.handle) == 0
+
+    g = hr.Graph(s, call)
+    for run in (g.launch, call, g.launch):
+        dc.upload(np.full(m * n, -7, np.int32))
+        run()
+        s.synchronize()
+        assert (dc.download(np.int32, (m, n)) == ref).all()
+    lib.ternix_hip_release_stream(s.handle)
+
+
 def test_gemm_plans_split_whole_blocks(lib):
     """Every plan over a range of sizes is described, and its workspace fits its splits (no launch)."""
     import ctypes
