@@ -1064,6 +1064,15 @@ hipError_t run_tile64(const int8_t* dA, const uint8_t* dWt, int32_t* dC, int M, 
         hipError_t e = hipSuccess;
         if (run_line_gemv(dA, dWt, dC, M, K, N, c, &e, os, ternix_hip::ActQuant{}, 1)) return e;
     }
+    // 17-32 rows, float output, short K: the GEMM's 32-row tiles where the row-major estimates say so (on MI355X,
+    // warm, quantised layers: 21x1536x3840 11.0 -> 8.8 us, 18x512x2816 9.7 -> 7.0, 20x768x512 8.7 -> 7.4; with a longer K
+    // this layout's own kernels are level or ahead, 17x2304x512 9.3 against 9.8, 20x12288x5120 16.4 against 17.7, as they
+    // are up to 16 rows).
+    const double mb = (double)K * (double)N / 4e6, mn = (double)M * (double)N * 1e-6;
+    if (M > 16 && M <= 32 && os.Y != nullptr && K >= 256 && K <= 2048 && mb <= 32.0 &&
+        ternix_hip::debug_get(ternix_hip::DBG_DEEP) < 0 && ternix_hip::debug_get(ternix_hip::DBG_SKINNY_WAVE) < 0 &&
+        few_rows_gemm_us(K, mb) < 0.95 * few_rows_float_us(M, K, mb, mn))
+        return run_gemm(dA, dWt, dC, M, K, N, c, os, 1);
     // The self-zeroing atomic plan below applies to int32 output up to 16 rows; where it does, it is
     // faster than the whole-K kernel (cold, one box, us: cfg1 4.80 -> 3.64, cfg2 up 5.10 -> 4.49, 4x4096x11008
     // 6.46 -> 6.32, 16x4096x11008 7.69 -> 7.31), which keeps the dequantising calls.
@@ -1527,21 +1536,12 @@ int ternix_hip_ffn_forward_tile64(float* dY, const float* dX, const float* dNorm
             return (int)run_tile64(q2, dWdT, reinterpret_cast<int32_t*>(dY), m, f, hd, ctx_of(st), os2);
         }
     }
-    if (m <= 16 && hd <= 4096) {
-        // RMSNorm + quantisation of x inside the gate/up GEMV (one launch, whole rows per workgroup).
-        ternix_hip::ActQuant aq1;
-        aq1.mode = 2;
-        aq1.X = dX;
-        aq1.G = dNormWeight;
-        aq1.eps = eps;
-        aq1.rs_out = rs1;
-        e = ternix_hip::launch_skinny_wave(nullptr, dWguT, scratch, m, hd, 2 * f, 16, 2, 1, hd / 64, nullptr, st, os1,
-                                           0, aq1, 1);
-    } else {
-        const int s = ternix_hip_rms_norm_quantize(q1, rs1, dX, dNormWeight, M, H, eps, stream);
-        if (s != 0) return s;
-        e = run_tile64(q1, dWguT, scratch, m, hd, 2 * f, ctx_of(st), os1);
-    }
+    // Otherwise separate launches.  (RMSNorm + quantisation inside the gate/up GEMV, every workgroup over whole rows,
+    // took 5-16 rows before; on MI355X, warm, us per block: 15 x 2560 x 9472 45.6 -> 25.2, 14 x 1536 x 1280 34.3 -> 15.5,
+    // 7 x 768 x 768 22.4 -> 14.0, 5 x 512 x 2816 19.7 -> 14.7.)
+    const int s = ternix_hip_rms_norm_quantize(q1, rs1, dX, dNormWeight, M, H, eps, stream);
+    if (s != 0) return s;
+    e = run_tile64(q1, dWguT, scratch, m, hd, 2 * f, ctx_of(st), os1);
     if (e != hipSuccess) return (int)e;
     e = ternix_hip::launch_quantize_rows(h, q2, rs2, m, f, st);
     if (e != hipSuccess) return (int)e;

@@ -78,3 +78,19 @@ def test_dequant_first_call_inside_capture(oracle, shape):
         s.synchronize()
         np.testing.assert_array_equal(dy.download(F32, (m, n)), y)
     lib.ternix_hip_release_stream(s.handle)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(17, 512, 768), (32, 2048, 1024), (32, 2176, 256), (16, 512, 768)], ids=lambda s: "x".join(map(str, s)))
+def test_tile64_few_rows_float(oracle, shape):
+    """Tile-64 weights, either side of the rules for the GEMM's 32-row tiles: the row-major layout's bits."""
+    lib = tx._load()
+    m, k, n = shape
+    print(f"tile-64 M={m} K={k} N={n}", flush=True)
+    a, wp, rs, (da, dw, drs) = _bufs(np.random.default_rng(sum(shape)), m, k, n)
+    dt, dy = hr.DeviceBuffer(wp.nbytes), hr.DeviceBuffer(4 * m * n)
+    assert tx.interleave_tile64_device(dt.value, dw.value, k, n) == 0
+    assert lib.ternix_hip_mul_mat_ternary_tile64_dequant(da.value, dt.value, dy.value, m, k, n, drs.value, 0.25, None) == 0
+    hr.synchronize()
+    ref = oracle.mm("scalar_mt", a, wp, n).astype(F32) * (rs * F32(0.25))[:, None]
+    np.testing.assert_array_equal(dy.download(F32, (m, n)), ref)
