@@ -5,9 +5,9 @@
 // weight (k, n) in bits 2*(n%4) of byte k*NB + n/4; 00 = 0, 01 = +1, 11 = -1 (10 decodes as -2,
 // like the reference's scalar and CUDA decode, src/mul_mat_ternary.cpp:53, src/cuda_kernels.cu:40).
 //
-// Every matmul kernel here feeds v_mfma_i32_16x16x64_i8.  The int8 MFMA reduces along K inside a
-// lane (lane l holds 16 K-consecutive bytes of one row of A and of one column of B, K-block l/16),
-// while the packed layout runs along N.  The kernels therefore
+// Every matmul kernel here feeds v_mfma_i32_16x16x64_i8 (gemm_pipe_kernel: 32x32x32).  The int8 MFMA reduces
+// along K inside a lane (lane l holds 16 K-consecutive bytes of one row of A and of one column of B, K-block
+// l/16, or l/32), while the packed layout runs along N.  The kernels therefore
 //   1. gather, per lane, one packed byte-column (= 4 output columns) over 16 consecutive k-rows:
 //      with the gfx950 transposing LDS read ds_read_b64_tr_b8 from a row-major LDS stage (the
 //      DMA-staged and wave-pipelined GEMVs, the pipelined GEMM), or with a 4x4 byte transpose in
@@ -22,7 +22,7 @@
 //   skinny_wave_kernel    M <= 32: 16-byte weight strips, per-wave DMA rings, one launch for K <= 4096
 //   skinny_dma_kernel     M <= 16, long K: 256-byte strips staged by DMA, split-K + reduce
 //   skinny_short/fast/generic_kernel  register-staged GEMVs (fallbacks, fused FFN prologue)
-//   gemm_pipe_kernel / gemm_fast_kernel / gemm_kernel  LDS-tiled MFMA GEMMs (M > 32)
+//   gemm_pipe_kernel / gemm_pipe16_kernel / gemm_kernel  LDS-tiled MFMA GEMMs (M > 32, and 4-32 rows of short K)
 //   splitk_reduce_kernel, pad_rows_kernel, quantize / dequant kernels: the steps around them
 //
 // Field decode.  Let x be 4 bytes (4 k-rows), each holding fields f0..f3 (bits 0-1 .. 6-7).
